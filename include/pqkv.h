@@ -361,6 +361,13 @@ int pqkv_prefill_attn(const void *q, int q_dtype, const float *R,
  * R [d][d] fp32 16-byte aligned, out [n][d] fp32/fp16. */
 int pqkv_dequantize(const uint8_t *blocks, const float *codebook, int n_bits, const float *R,
                     void *out, int out_dtype, int64_t n, int d, void *stream);
+/* The same for n_outer rows of n_inner vectors: row o starts
+ * o * blocks_outer_stride bytes into blocks (at least a row's bytes)
+ * and o * out_outer_stride elements into out: every head of a cache longer
+ * than its valid positions in one launch. */
+int pqkv_dequantize_rows(const uint8_t *blocks, int64_t blocks_outer_stride, const float *codebook, int n_bits,
+                         const float *R, void *out, int out_dtype, int64_t out_outer_stride, int64_t n_outer,
+                         int64_t n_inner, int d, void *stream);
 
 /* ---- layout converters ---------------------------------------------------
  * SoA (the reference kernels' format: packed u8 [n][d/2] + fp32 radius [n],

@@ -1128,18 +1128,29 @@ int pqkv_prefill_attn_paged(const void *q, int q_dtype, const float *R, const ui
                                 out_dtype, workspace, workspace_bytes, stream, &pg);
 }
 
-int pqkv_dequantize(const uint8_t *blocks, const float *codebook, int n_bits, const float *R, void *out,
-                    int out_dtype, int64_t n, int d, void *stream) {
-  if (n < 0) return fail(PQKV_ERR_INVALID, "dequantize: n < 0");
+int pqkv_dequantize_rows(const uint8_t *blocks, int64_t blocks_outer_stride, const float *codebook, int n_bits,
+                         const float *R, void *out, int out_dtype, int64_t out_outer_stride, int64_t n_outer,
+                         int64_t n_inner, int d, void *stream) {
+  if (n_outer < 0 || n_inner < 0) return fail(PQKV_ERR_INVALID, "dequantize: n < 0");
   if (!supported_d(d) || !supported_bits(n_bits)) return fail(PQKV_ERR_UNSUPPORTED, "dequantize: d=%d bits=%d", d, n_bits);
   if (!float_dtype(out_dtype)) return fail(PQKV_ERR_UNSUPPORTED, "dequantize: dtype %d", out_dtype);
-  if (n == 0) return PQKV_OK;
+  if (n_outer == 0 || n_inner == 0) return PQKV_OK;
+  if (n_outer > 1 && (blocks_outer_stride < n_inner * pqkv_vector_bytes(d, n_bits) ||
+                      out_outer_stride < n_inner * d))
+    return fail(PQKV_ERR_INVALID, "dequantize: rows %lld bytes (out %lld elements) apart overlap",
+                (long long)blocks_outer_stride, (long long)out_outer_stride);
   if (!blocks || !codebook || !R || !out) return fail(PQKV_ERR_INVALID, "dequantize: null pointer");
   if ((uintptr_t)R % 16) return fail(PQKV_ERR_INVALID, "dequantize: R must be 16-byte aligned");
   const int tok = pqkv::prof_begin("dequantize", (hipStream_t)stream);
-  const hipError_t e = pqkv::launch_dequantize(blocks, codebook, n_bits, R, out, out_dtype, n, d, (hipStream_t)stream);
+  const hipError_t e = pqkv::launch_dequantize(blocks, blocks_outer_stride, codebook, n_bits, R, out, out_dtype,
+                                               out_outer_stride, n_outer, n_inner, d, (hipStream_t)stream);
   pqkv::prof_end(tok, (hipStream_t)stream);
   return hip_status(e, "dequantize launch");
+}
+
+int pqkv_dequantize(const uint8_t *blocks, const float *codebook, int n_bits, const float *R, void *out,
+                    int out_dtype, int64_t n, int d, void *stream) {
+  return pqkv_dequantize_rows(blocks, 0, codebook, n_bits, R, out, out_dtype, 0, 1, n, d, stream);
 }
 
 int pqkv_soa_to_blocks(const uint8_t *packed, const float *radius, uint8_t *blocks, int64_t n, int d,

@@ -49,7 +49,7 @@ __device__ __forceinline__ uint16_t radius_half_bits(float r) {
 struct FastDiv {
   uint32_t d, m;
   int s1, s2;
-  __device__ explicit FastDiv(uint32_t div) : d(div) {
+  __host__ __device__ explicit FastDiv(uint32_t div) : d(div) {
     int l = 0;
     while (l < 32 && (1ull << l) < div) ++l;
     m = (uint32_t)((((uint64_t)1 << 32) * (((uint64_t)1 << l) - div)) / div + 1);

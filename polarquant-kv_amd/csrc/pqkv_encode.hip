@@ -195,26 +195,7 @@ struct RowsSource {
     return x[sq * s_s + h * s_h + iq * s_q + j];
   }
 };
-// Block-encoded vectors (block_pq4 / block_pq2): r16 * c[code], the rotated
-// reconstruction the attention kernels use.
-template <int D, int BITS>
-struct BlockSource {
-  const uint8_t *blocks;
-  const float *cb;
-  __device__ __forceinline__ float operator()(int64_t v, int j) const {
-    constexpr int VB = vector_bytes(D, BITS);
-    const uint8_t *vec = blocks + v * VB;
-    const float r = half_bits_to_float(*(const uint16_t *)vec);
-    const int per = 8 / BITS;                              // codes per byte
-    const uint8_t byte = vec[qs_offset(j / per, BITS)];
-    const int code = (byte >> (BITS * (j % per))) & ((1 << BITS) - 1);
-    return r * cb[code];
-  }
-};
-
-// SAT16: fp16 output saturates at +-65504 like the reference's decompress
-// (decompress_kernel.py:52-55, clamp(-65504, 65504).half()).
-template <int D, bool INVERSE, typename SRC, typename TOUT, bool SAT16 = false>
+template <int D, bool INVERSE, typename SRC, typename TOUT>
 __global__ void __launch_bounds__(256) rotate_kernel(const SRC src, const float *__restrict__ R,
                                                      TOUT *__restrict__ y, int64_t n, float out_scale) {
   constexpr int RP = D + 4;
@@ -273,9 +254,7 @@ __global__ void __launch_bounds__(256) rotate_kernel(const SRC src, const float 
     }
     const int64_t v = base + g;
     if (v < n) {
-      float o = acc * out_scale;
-      if (SAT16) o = o > 65504.0f ? 65504.0f : (o < -65504.0f ? -65504.0f : o);
-      y[v * D + c0 + jj] = (TOUT)o;
+      y[v * D + c0 + jj] = (TOUT)(acc * out_scale);
     }
     __syncthreads();
   }
@@ -356,8 +335,22 @@ __global__ void __launch_bounds__(256) rotate2_kernel(const TIN *__restrict__ x,
   }
 }
 
+// Many vectors (on a 16-byte boundary) go to the fp32 matrix cores, the same
+// bits. Measured crossover (fp16 -> fp32, replayed graphs): d = 128 3.7 us here
+// against 4.7 us there at 1024 vectors, 5.0 against 4.8 at 2048, 12.1 against
+// 5.3 at 8192, 392 against 103 at 400 000; d = 64 2.7 against 3.1 at 2048, 3.6
+// against 3.2 at 4096, 107 against 32 at 400 000. Below it the launch spreads
+// over too few compute units there (32 or 64 vectors per workgroup, 8 here).
+static bool rotate_mfma_ok(const void *x, int64_t n, int d) {
+  return n >= (d == 128 ? 2048 : 4096) && (uintptr_t)x % 16 == 0;
+}
+
 hipError_t launch_rotate2(const void *x, int x_dtype, const float *R, const float *M, float *y, float *z, int64_t n,
                           int d, float sy, float sz, hipStream_t s) {
+  if (rotate_mfma_ok(x, n, d)) {
+    const hipError_t e = launch_rotate_mfma(x, x_dtype, R, y, 0, n, d, 0, sy, s);
+    return e != hipSuccess ? e : launch_rotate_mfma(y, 0, M, z, 0, n, d, 0, sz, s);
+  }
   const int64_t grid = (n + kRot2Vec - 1) / kRot2Vec;
   if (grid < 1 || grid > 0x7fffffff) return hipErrorInvalidValue;
   if (d == 128) {
@@ -649,6 +642,8 @@ static void rotate_dispatch(const void *x, int xt, const float *R, void *y, int 
 hipError_t launch_rotate_rows(const float *x, int64_t s_q, int64_t s_h, int64_t s_s, int n_q, int Hq, int n_seq,
                               const float *R, float *y, int d, float out_scale, hipStream_t s) {
   const int64_t n = (int64_t)n_seq * n_q * Hq;
+  if (rotate_mfma_ok(x, n, d) && s_q % 4 == 0 && s_h % 4 == 0 && s_s % 4 == 0)
+    return launch_rotate_rows_mfma(x, s_q, s_h, s_s, n_q, Hq, n_seq, R, y, d, out_scale, s);
   const RowsSource src{x, s_q, s_h, s_s, n_q, Hq};
   if (d == 128) {
     const dim3 grid(grid_for(n, kRotVec, 2048), 128 / kRotCols);
@@ -657,24 +652,6 @@ hipError_t launch_rotate_rows(const float *x, int64_t s_q, int64_t s_h, int64_t 
     const dim3 grid(grid_for(n, kRotVec, 2048), 64 / kRotCols);
     rotate_kernel<64, false, RowsSource, float><<<grid, 256, 0, s>>>(src, R, y, n, out_scale);
   }
-  return hipGetLastError();
-}
-
-template <int D, int BITS>
-static void dequant_dispatch(const uint8_t *blocks, const float *cb, const float *R, void *y, int yt, int64_t n,
-                             hipStream_t s) {
-  const dim3 grid(grid_for(n, kRotVec, 4096), D / kRotCols);
-  using S = BlockSource<D, BITS>;
-  if (yt == 0) rotate_kernel<D, true, S, float><<<grid, 256, 0, s>>>(S{blocks, cb}, R, (float *)y, n, 1.0f);
-  else rotate_kernel<D, true, S, half_t, true><<<grid, 256, 0, s>>>(S{blocks, cb}, R, (half_t *)y, n, 1.0f);
-}
-
-hipError_t launch_dequantize(const uint8_t *blocks, const float *codebook, int bits, const float *R, void *y,
-                             int y_dtype, int64_t n, int d, hipStream_t s) {
-  if (d == 128 && bits == 4) dequant_dispatch<128, 4>(blocks, codebook, R, y, y_dtype, n, s);
-  else if (d == 128) dequant_dispatch<128, 2>(blocks, codebook, R, y, y_dtype, n, s);
-  else if (bits == 4) dequant_dispatch<64, 4>(blocks, codebook, R, y, y_dtype, n, s);
-  else dequant_dispatch<64, 2>(blocks, codebook, R, y, y_dtype, n, s);
   return hipGetLastError();
 }
 
@@ -689,6 +666,7 @@ hipError_t launch_rotate(const void *x, int x_dtype, const float *R, void *y, in
     else scale_kernel<<<grid, 256, 0, s>>>((const half_t *)x, (half_t *)y, m, out_scale);
     return hipGetLastError();
   }
+  if (rotate_mfma_ok(x, n, d)) return launch_rotate_mfma(x, x_dtype, R, y, y_dtype, n, d, inverse, out_scale, s);
   if (d == 128) {
     if (inverse) rotate_dispatch<128, true>(x, x_dtype, R, y, y_dtype, n, out_scale, s);
     else rotate_dispatch<128, false>(x, x_dtype, R, y, y_dtype, n, out_scale, s);

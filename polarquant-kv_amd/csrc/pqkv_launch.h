@@ -198,10 +198,18 @@ hipError_t launch_rotate(const void *x, int x_dtype, const float *R, void *y, in
 // chains of launch_rotate.
 hipError_t launch_rotate_rows(const float *x, int64_t s_q, int64_t s_h, int64_t s_s, int n_q, int Hq, int n_seq,
                               const float *R, float *y, int d, float out_scale, hipStream_t s);
-// y = (r16 c[code]) R for n block-encoded vectors (inverse rotation, one
-// FMA chain per output as in launch_rotate); fp16 output saturates.
-hipError_t launch_dequantize(const uint8_t *blocks, const float *codebook, int bits, const float *R, void *y,
-                             int y_dtype, int64_t n, int d, hipStream_t s);
+// The same rotations on the fp32 matrix cores, for many vectors (x on a
+// 16-byte boundary, strides in multiples of 16 bytes): the same bits.
+hipError_t launch_rotate_mfma(const void *x, int x_dtype, const float *R, void *y, int y_dtype, int64_t n, int d,
+                              int inverse, float out_scale, hipStream_t s);
+hipError_t launch_rotate_rows_mfma(const float *x, int64_t s_q, int64_t s_h, int64_t s_s, int n_q, int Hq, int n_seq,
+                                   const float *R, float *y, int d, float out_scale, hipStream_t s);
+// y = (r16 c[code]) R for n_outer rows of n_inner block-encoded vectors, rows
+// blocks_outer_stride bytes (y_outer_stride elements) apart (inverse rotation,
+// one FMA chain per output as in launch_rotate); fp16 output saturates.
+hipError_t launch_dequantize(const uint8_t *blocks, int64_t blocks_outer_stride, const float *codebook, int bits,
+                             const float *R, void *y, int y_dtype, int64_t y_outer_stride, int64_t n_outer,
+                             int64_t n_inner, int d, hipStream_t s);
 hipError_t launch_encode_exact(const EncodeArgs &a, int x_dtype, hipStream_t s);
 // Register-blocked form of the exact encoder (same rotation, same indices)
 // for inputs it reads in 16-byte pieces, without QJL signs; the exact

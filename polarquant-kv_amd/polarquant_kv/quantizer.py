@@ -219,29 +219,23 @@ def dequantize(cache: PQCache, rotation_matrix: torch.Tensor | None, out_dtype=t
         return out
     lib = _lib.lib()
     stream = _lib.stream_of(out)
-    for b in range(B):
-        for h, bits in enumerate(cache.head_bits()):
-            vb = vector_bytes(d, bits)
-            if cache.mixed:
-                src = cache.blocks[b].data_ptr() + cache.head_offset(h)
-                cb = cache.codebooks[h] if cache.codebooks.dim() == 2 else cache.codebooks
-            else:
-                if h > 0:
-                    continue
-                # uniform widths: every head of the batch row in one call when
-                # the rows are contiguous (S == max_seq_len), else per head
-                cb = cache.codebooks
-                if S == cache.max_seq_len:
-                    _lib.check(lib.pqkv_dequantize(cache.blocks[b].data_ptr(), cb.data_ptr(), bits, R.data_ptr(),
-                                                   out[b].data_ptr(), _lib.dtype_code(out_dtype), H * S, d, stream))
-                    continue
-                for hh in range(H):
-                    _lib.check(lib.pqkv_dequantize(cache.blocks[b, hh].data_ptr(), cb.data_ptr(), bits,
-                                                   R.data_ptr(), out[b, hh].data_ptr(), _lib.dtype_code(out_dtype),
-                                                   S, d, stream))
-                continue
-            _lib.check(lib.pqkv_dequantize(src, cb.data_ptr(), bits, R.data_ptr(), out[b, h].data_ptr(),
-                                           _lib.dtype_code(out_dtype), S, d, stream))
+    code = _lib.dtype_code(out_dtype)
+    if not cache.mixed:
+        # every (batch, head) row of the cache, S_max vectors apart, in one
+        # launch (one per batch row where the batch stride is its own)
+        sb, sh = cache.blocks.stride(0), cache.blocks.stride(1)
+        rows, batches = (B * H, 1) if sb == H * sh else (H, B)
+        for b in range(batches):
+            _lib.check(lib.pqkv_dequantize_rows(cache.blocks[b].data_ptr(), sh, cache.codebooks.data_ptr(),
+                                                cache.n_bits, R.data_ptr(), out[b].data_ptr(), code, S * d, rows, S, d,
+                                                stream))
+        return out
+    for h, bits in enumerate(cache.head_bits()):
+        # one head of every batch row per launch
+        cb = cache.codebooks[h] if cache.codebooks.dim() == 2 else cache.codebooks
+        _lib.check(lib.pqkv_dequantize_rows(cache.blocks.data_ptr() + cache.head_offset(h), cache.blocks.stride(0),
+                                            cb.data_ptr(), bits, R.data_ptr(), out[:, h].data_ptr(), code, H * S * d,
+                                            B, S, d, stream))
     return out
 
 

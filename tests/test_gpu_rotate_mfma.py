@@ -1,0 +1,96 @@
+"""Rotations and decodes of many vectors on the fp32 matrix cores: every output
+bit equals the one-FMA-chain form (the C oracle, and the small-launch kernel on
+special values), at the sizes around the dispatch line, step remainders, row
+strides and odd alignments."""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as OC
+from oracle import oracle as O
+from polarquant_kv import _lib, quantizer
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _rotate(x, R, inverse, out):
+    _lib.check(_lib.lib().pqkv_rotate(x.data_ptr(), _lib.dtype_code(x.dtype), R.data_ptr(), out.data_ptr(),
+                                      _lib.dtype_code(out.dtype), x.shape[0], x.shape[1], inverse, _lib.stream_of(x)))
+    return out
+
+
+def _bits(t):
+    return t.contiguous().view(torch.int32 if t.dtype == torch.float32 else torch.int16)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("inverse", [0, 1])
+@pytest.mark.parametrize("extra", [-1, 0, 1, 31, 33, 4095])
+def test_rotate_bits_around_the_line(d, inverse, extra):
+    n = (2048 if d == 128 else 4096) + extra
+    print(f"rotate d={d} inverse={inverse} n={n}", flush=True)
+    g = torch.Generator().manual_seed(n + d)
+    x = torch.randn(n, d, generator=g)
+    x[0], x[1], x[2] = 0.0, x[1] * 2.0 ** -140, x[2] * 2.0 ** 100
+    R = torch.from_numpy(O.rotation_matrix(d, 42).astype(np.float32))
+    want = OC.c_rotate_fma(x.numpy(), R.numpy(), inverse=bool(inverse))
+    Rd = R.to(DEV)
+    got = _rotate(x.to(DEV), Rd, inverse, torch.empty(n, d, device=DEV))
+    assert np.array_equal(got.cpu().numpy().view(np.uint32), want.view(np.uint32))
+    xh = x.half()
+    want16 = OC.c_rotate_fma(xh.float().numpy(), R.numpy(), inverse=bool(inverse))
+    got16 = _rotate(xh.to(DEV), Rd, inverse, torch.empty(n, d, device=DEV, dtype=torch.float16))
+    with np.errstate(over="ignore"):
+        assert np.array_equal(got16.cpu().numpy().view(np.uint16), want16.astype(np.float16).view(np.uint16))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_rotate_special_values_and_odd_alignment(d):
+    """Infinities and NaN as in the small launches; an x off a 16-byte boundary
+    still takes the general kernel."""
+    n = 5000
+    x = torch.randn(n + 1, d)
+    x[7, 3], x[8, 5], x[9, d - 1], x[10, 0] = float("inf"), float("-inf"), float("nan"), 3e38
+    R = torch.from_numpy(O.rotation_matrix(d, 42).astype(np.float32)).to(DEV)
+    flat = torch.empty((n + 1) * d + 1, device=DEV)
+    for off in (0, 1):
+        xd = flat[off:off + n * d].view(n, d)
+        xd.copy_(x[:n])
+        many = _rotate(xd, R, 0, torch.empty(n, d, device=DEV))
+        few = torch.cat([_rotate(xd[i:i + 500], R, 0, torch.empty(500, d, device=DEV)) for i in range(0, n, 500)])
+        nan = torch.isnan(few)
+        assert torch.equal(torch.isnan(many), nan)
+        assert torch.equal(_bits(many)[~nan], _bits(few)[~nan])
+
+
+@pytest.mark.parametrize("d,bits", [(64, 2), (64, 4), (128, 2), (128, 4)])
+@pytest.mark.parametrize("B,H,S,cap", [(1, 1, 1, 1), (2, 3, 33, 64), (3, 2, 700, 701), (1, 4, 2049, 2049)])
+def test_dequantize_rows_bits(d, bits, B, H, S, cap):
+    """Every head of a cache longer than its valid positions in one launch,
+    and a batch stride of its own; a mixed cache's heads as the uniform ones'."""
+    print(f"dequantize d={d} bits={bits} B={B} H={H} S={S}", flush=True)
+    rng = np.random.default_rng(d + bits + S)
+    idx = rng.integers(0, 1 << bits, (B * H * cap, d)).astype(np.uint8)
+    r = rng.lognormal(0, 2, B * H * cap).astype(np.float32)
+    blocks = O.pack_blocks(r, idx, bits)
+    cb = O.lloyd_max_codebook(d, bits)[0]
+    R = O.rotation_matrix(d, 42).astype(np.float32)
+    r16, idx2 = O.unpack_blocks(blocks, d, bits)
+    xr = (r16.astype(np.float32)[:, None] * cb[idx2]).astype(np.float32)
+    want = OC.c_rotate_fma(xr, R, inverse=True).reshape(B, H, cap, d)[:, :, :S]
+    cache = quantizer.allocate_cache(B, H, cap, d, bits, DEV)
+    cache.blocks.copy_(torch.from_numpy(blocks).view(B, H, cap, -1))
+    cache.seq_len = S
+    Rt = torch.from_numpy(R).to(DEV)
+    got = quantizer.dequantize(cache, Rt, torch.float32)
+    assert np.array_equal(got.cpu().numpy().view(np.uint32), want.view(np.uint32))
+    wide = torch.zeros(B, H + 1, cap, cache.blocks.shape[-1], dtype=torch.uint8, device=DEV)
+    wide[:, :H] = cache.blocks
+    cache.blocks = wide[:, :H]
+    assert torch.equal(_bits(quantizer.dequantize(cache, Rt, torch.float32)), _bits(got))
+    mixed = quantizer.allocate_cache(B, H, cap, d, (bits,) * H, DEV)
+    mixed.blocks.copy_(wide[:, :H].reshape(B, -1))
+    mixed.seq_len = S
+    assert torch.equal(_bits(quantizer.dequantize(mixed, Rt, torch.float32)), _bits(got))
