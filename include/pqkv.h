@@ -275,7 +275,8 @@ int pqkv_group_decompress(const float *radius, const uint8_t *codes, const float
  * packed as the reference packs them: 4-bit d_pad/2 bytes (coordinate 2i
  * low nibble), 2-bit d_pad/4 bytes (v0 | v1<<2 | v2<<4 | v3<<6), every
  * other width one byte per code. x fp32 / fp16 / bf16 [n][d]; R [d][d] fp32
- * and Rt = R^T (both device); 1 <= d <= 256, 2 <= n_bits <= 8. residual
+ * and Rt = R^T (both device; either may be NULL without a residual, which
+ * needs R); 1 <= d <= 256, 2 <= n_bits <= 8. residual
  * (nullable, needs R) receives the QJL residual e = (y - (code s + lo)
  * max(r, 1e-30)) R [n][d] fp32 with the unrounded lo and s
  * (compress_kernel.py:166-175). Replaces compress_gpu. */

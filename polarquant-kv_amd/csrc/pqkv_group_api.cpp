@@ -74,7 +74,7 @@ int pqkv_group_gpu_compress(const void *x, int x_dtype, const float *R, const fl
   if (!in_dtype_ok(x_dtype) || !param_dtype_ok(param_dtype))
     return fail(PQKV_ERR_UNSUPPORTED, "group_gpu_compress: dtype x=%d params=%d", x_dtype, param_dtype);
   if (n == 0) return PQKV_OK;
-  if (!x || !Rt || !radius || !codes || !mins || !scales || (residual && !R))
+  if (!x || (!Rt && !R) || !radius || !codes || !mins || !scales || (residual && !R))
     return fail(PQKV_ERR_INVALID, "group_gpu_compress: null pointer");
   return hip_status(pqkv::launch_group_gpu_compress(x, x_dtype, Rt, R, n, d, n_bits, group_size, radius, codes, mins,
                                                     scales, param_dtype, residual, (hipStream_t)stream),

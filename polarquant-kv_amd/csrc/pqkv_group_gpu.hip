@@ -71,7 +71,7 @@ __device__ __forceinline__ int code_at(const uint8_t *row, int cb, int j) {
 
 // ---------------------------------------------------------------------------
 // compress: one wave per vector. Rt = R^T ([k][j] = R[j][k]) so that lane j's
-// reads of a row of R are coalesced across the wave.
+// reads of a row of R are coalesced across the wave (null: R's own rows).
 __global__ void __launch_bounds__(kGW * 64)
     group_gpu_compress_kernel(const void *x, int x_dtype, const float *Rt, const float *R, int64_t n, int d, int bits,
                               int gs, void *radius, uint8_t *codes, void *mins, void *scales, int pdt,
@@ -99,7 +99,9 @@ __global__ void __launch_bounds__(kGW * 64)
       y[i] = 0.0f;
       if (j < d) {
         float acc = 0.0f;
-        for (int k = 0; k < d; ++k) acc = __builtin_fmaf(xs[w][k], Rt[(int64_t)k * d + j], acc);
+        const float *rp = Rt ? Rt + j : R + (int64_t)j * d;
+        const int rs = Rt ? d : 1;
+        for (int k = 0; k < d; ++k) acc = __builtin_fmaf(xs[w][k], rp[(int64_t)k * rs], acc);
         y[i] = acc;
         sq += (double)acc * (double)acc;
       }
@@ -809,6 +811,9 @@ hipError_t launch_group_gpu_compress(const void *x, int x_dtype, const float *Rt
                                      int bits, int gs, void *radius, uint8_t *codes, void *mins, void *scales,
                                      int pdt, float *resid, hipStream_t s) {
   if (d < 1 || d > kGMax || gs < 1 || gs > d) return hipErrorInvalidValue;
+  if (n <= 0) return hipSuccess;
+  if (group_compress_mfma_ok(x, R, Rt, d, gs, codes, resid))
+    return launch_group_compress_mfma(x, x_dtype, Rt, R, n, d, bits, gs, radius, codes, mins, scales, pdt, resid, s);
   group_gpu_compress_kernel<<<grid_for(n), kGW * 64, 0, s>>>(x, x_dtype, Rt, R, n, d, bits, gs, radius, codes, mins,
                                                              scales, pdt, resid);
   return hipGetLastError();

@@ -271,6 +271,13 @@ hipError_t launch_group_decompress(const float *radius, const uint8_t *codes, co
 hipError_t launch_group_gpu_compress(const void *x, int x_dtype, const float *Rt, const float *R, int64_t n, int d,
                                      int bits, int gs, void *radius, uint8_t *codes, void *mins, void *scales,
                                      int pdt, float *resid, hipStream_t s);
+// The same on the fp32 matrix cores (same bits): d = 64 or 128, gs a power of
+// two from 8, x, R and codes on 16-byte boundaries. R may be null without resid.
+bool group_compress_mfma_ok(const void *x, const float *R, const float *Rt, int d, int gs, const uint8_t *codes,
+                            const float *resid);
+hipError_t launch_group_compress_mfma(const void *x, int x_dtype, const float *Rt, const float *R, int64_t n, int d,
+                                      int bits, int gs, void *radius, uint8_t *codes, void *mins, void *scales,
+                                      int pdt, float *resid, hipStream_t s);
 hipError_t launch_group_gpu_decompress(const void *radius, const uint8_t *codes, const void *mins,
                                        const void *scales, int pdt, const float *R, int64_t n, int d, int bits,
                                        int gs, void *out, int out_dtype, hipStream_t s);

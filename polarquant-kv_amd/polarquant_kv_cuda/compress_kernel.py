@@ -70,20 +70,23 @@ def _transposed(R: torch.Tensor) -> torch.Tensor:
 
 
 def empty_cache(batch: int, heads: int, seq: int, d: int, n_bits: int, group_size: int, device, jl_dim: int = 0,
-                max_seq_len: int | None = None) -> CompressedKVCacheGPU:
-    """A group-format cache of max_seq_len (default seq) positions, seq_len = seq."""
+                max_seq_len: int | None = None, zero: bool = True) -> CompressedKVCacheGPU:
+    """A group-format cache of max_seq_len (default seq) positions, seq_len =
+    seq; zero=False leaves its fields uninitialised, for a caller that writes
+    every position."""
+    new = torch.zeros if zero else torch.empty
     S = seq if max_seq_len is None else max_seq_len
     ng = math.ceil(d / group_size) if d > 0 else 0
     pd = _packed_dim(ng * group_size, n_bits)
     signs = norms = None
     if jl_dim:
-        signs = torch.zeros(batch, heads, S, (jl_dim + 7) // 8, dtype=torch.uint8, device=device)
-        norms = torch.zeros(batch, heads, S, dtype=torch.float16, device=device)
+        signs = new(batch, heads, S, (jl_dim + 7) // 8, dtype=torch.uint8, device=device)
+        norms = new(batch, heads, S, dtype=torch.float16, device=device)
     return CompressedKVCacheGPU(
-        radius=torch.zeros(batch, heads, S, dtype=torch.float16, device=device),
-        quantized_direction=torch.zeros(batch, heads, S, pd, dtype=torch.uint8, device=device),
-        group_mins=torch.zeros(batch, heads, S, ng, dtype=torch.float16, device=device),
-        group_scales=torch.zeros(batch, heads, S, ng, dtype=torch.float16, device=device),
+        radius=new(batch, heads, S, dtype=torch.float16, device=device),
+        quantized_direction=new(batch, heads, S, pd, dtype=torch.uint8, device=device),
+        group_mins=new(batch, heads, S, ng, dtype=torch.float16, device=device),
+        group_scales=new(batch, heads, S, ng, dtype=torch.float16, device=device),
         qjl_signs=signs, residual_norms=norms, n_bits=n_bits, group_size=group_size, original_dim=d,
         seq_len=seq, max_seq_len=S)
 
@@ -99,7 +102,9 @@ def _compress_rows(x: torch.Tensor, R: torch.Tensor, n_bits: int, group_size: in
     code = {torch.float16: _lib.F16, torch.float32: _lib.F32, torch.bfloat16: _lib.BF16}[x.dtype]
     Rf = R.to(device=x.device, dtype=torch.float32).contiguous()
     resid = torch.empty(n, d, dtype=torch.float32, device=x.device) if jl_matrix is not None else None
-    _lib.check(lib.pqkv_group_gpu_compress(x.data_ptr(), code, Rf.data_ptr(), _transposed(Rf).data_ptr(), n, d,
+    # the matrix-core encoder reads R alone; the general one is faster with R^T
+    Rt = None if d in (64, 128) and group_size in (8, 16, 32, 64, 128) and x.data_ptr() % 16 == 0 else _transposed(Rf)
+    _lib.check(lib.pqkv_group_gpu_compress(x.data_ptr(), code, Rf.data_ptr(), _lib.ptr(Rt), n, d,
                                            n_bits, group_size, out["radius"].data_ptr(), out["codes"].data_ptr(),
                                            out["mins"].data_ptr(), out["scales"].data_ptr(), _lib.F16,
                                            _lib.ptr(resid), stream))
@@ -129,7 +134,7 @@ def compress_gpu(kv: torch.Tensor, rotation_matrix: torch.Tensor, n_bits: int = 
     B, H, S, d = kv.shape
     _validate_params(n_bits, group_size, d)
     m = 0 if jl_matrix is None else int(jl_matrix.shape[0])
-    cache = empty_cache(B, H, S, d, n_bits, group_size, kv.device, jl_dim=m)
+    cache = empty_cache(B, H, S, d, n_bits, group_size, kv.device, jl_dim=m, zero=False)
     out = {"radius": cache.radius, "codes": cache.quantized_direction, "mins": cache.group_mins,
            "scales": cache.group_scales, "signs": cache.qjl_signs, "norms": cache.residual_norms}
     _compress_rows(kv.reshape(-1, d).contiguous(), rotation_matrix, n_bits, group_size, jl_matrix, out)
