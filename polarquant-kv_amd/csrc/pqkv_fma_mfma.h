@@ -61,45 +61,56 @@ __device__ __forceinline__ void chain_load_columns(const float *__restrict__ R, 
 // This lane's operands of row j of R (forward rotation): r[s] =
 // R[j][2 s + half]. A workgroup of 256 threads reads R in runs (a lane reading
 // its own row would touch 32 lines per load) and hands the rows out through
-// `lds` (64 staged rows), 64 rows at a time; every thread calls it, and the
-// reads of `lds` are done (behind an LDS barrier of its own) when it returns.
+// LDS, 64 rows at a time: issue() starts the loads, and spread(), which every
+// thread calls, hands the rows out through `lds` (64 staged rows, whose last
+// reads are done, behind an LDS barrier of its own, when it returns).
+template <int D>
+struct ChainRows {
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  static constexpr int kPieces = 64 * (D / 8) / 256;   // 8-coordinate pieces per thread and pass
+  f4 w[D / 64][kPieces][2];
+  __device__ __forceinline__ void issue(const float *__restrict__ R, int tid) {
+#pragma unroll
+    for (int p = 0; p < D / 64; ++p)
+#pragma unroll
+      for (int u = 0; u < kPieces; ++u) {
+        const f4 *src = (const f4 *)(R + (64 * p) * D + 8 * (tid + 256 * u));
+        w[p][u][0] = src[0];
+        w[p][u][1] = src[1];
+      }
+  }
+  __device__ __forceinline__ void spread(int tid, int j, int half, float *lds, float (&r)[D / 2]) const {
+    constexpr int PITCH = ChainRow<D>::kPitch;
+#pragma unroll
+    for (int p = 0; p < D / 64; ++p) {
+      if (p) lds_barrier();
+#pragma unroll
+      for (int u = 0; u < kPieces; ++u) {
+        const int item = tid + 256 * u;
+        const float o[8] = {w[p][u][0][0], w[p][u][0][1], w[p][u][0][2], w[p][u][0][3],
+                            w[p][u][1][0], w[p][u][1][1], w[p][u][1][2], w[p][u][1][3]};
+        chain_put8<D>(lds + (item / (D / 8)) * PITCH, item % (D / 8), o);
+      }
+      lds_barrier();
+      if (j / 64 == p) {
+        const float *row = lds + (j % 64) * PITCH + half * (D / 2);
+#pragma unroll
+        for (int s4 = 0; s4 < D / 8; ++s4) {
+          const f4 v = *(const f4 *)(row + 4 * s4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) r[4 * s4 + e] = v[e];
+        }
+      }
+    }
+    lds_barrier();
+  }
+};
 template <int D>
 __device__ __forceinline__ void chain_load_rows(const float *__restrict__ R, int tid, int j, int half, float *lds,
                                                 float (&r)[D / 2]) {
-  typedef float f4 __attribute__((ext_vector_type(4)));
-  constexpr int PIECES = 64 * (D / 8) / 256;   // 8-coordinate pieces per thread and pass
-  constexpr int PITCH = ChainRow<D>::kPitch;
-  f4 w[D / 64][PIECES][2];
-#pragma unroll
-  for (int p = 0; p < D / 64; ++p)
-#pragma unroll
-    for (int u = 0; u < PIECES; ++u) {
-      const f4 *src = (const f4 *)(R + (64 * p) * D + 8 * (tid + 256 * u));
-      w[p][u][0] = src[0];
-      w[p][u][1] = src[1];
-    }
-#pragma unroll
-  for (int p = 0; p < D / 64; ++p) {
-    if (p) lds_barrier();
-#pragma unroll
-    for (int u = 0; u < PIECES; ++u) {
-      const int item = tid + 256 * u;
-      const float o[8] = {w[p][u][0][0], w[p][u][0][1], w[p][u][0][2], w[p][u][0][3],
-                          w[p][u][1][0], w[p][u][1][1], w[p][u][1][2], w[p][u][1][3]};
-      chain_put8<D>(lds + (item / (D / 8)) * PITCH, item % (D / 8), o);
-    }
-    lds_barrier();
-    if (j / 64 == p) {
-      const float *row = lds + (j % 64) * PITCH + half * (D / 2);
-#pragma unroll
-      for (int s4 = 0; s4 < D / 8; ++s4) {
-        const f4 v = *(const f4 *)(row + 4 * s4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[4 * s4 + e] = v[e];
-      }
-    }
-  }
-  lds_barrier();
+  ChainRows<D> rows;
+  rows.issue(R, tid);
+  rows.spread(tid, j, half, lds, r);
 }
 
 }  // namespace pqkv
