@@ -864,6 +864,12 @@ size_t pqkv_prefill_workspace_bytes(int B, int Hq, int Hkv, int Sq, int S, int d
   return 3 * align256((size_t)B * Hq * Sq * d * 4);
 }
 
+size_t pqkv_prefill_workspace_preferred_bytes(int B, int Hq, int Hkv, int Sq, int S, int d, int qjl) {
+  const size_t n = pqkv_prefill_workspace_bytes(B, Hq, Hkv, Sq, S, d);
+  if (n == 0 || Hkv <= 0 || Hq % Hkv || Hq / Hkv > pqkv::prefill_rows_per_block(qjl != 0)) return n;
+  return n + pqkv::prefill_plan(B, Hq, Hkv, Sq, S, d, qjl != 0, true).bytes(d);
+}
+
 int pqkv_prefill_attn(const void *q, int q_dtype, const float *R, const uint8_t *k_cache, const uint8_t *v_cache,
                       const float *k_codebooks, const float *v_codebooks, int k_bits, int v_bits,
                       const int *k_head_bits, const int *v_head_bits, const uint8_t *qjl_signs, const float *p_rot,
@@ -925,11 +931,16 @@ int prefill_attn_run(const void *q, int q_dtype, const float *R, const uint8_t *
   }
   if ((pg ? (!pg->k_pages || !pg->v_pages) : (!k_cache || !v_cache)) || !k_codebooks || !v_codebooks)
     return fail(PQKV_ERR_INVALID, "prefill: null cache or codebook");
+  const int64_t nvec = (int64_t)B * Hq * Sq;
+  const size_t arr = align256((size_t)nvec * d * 4);
   const size_t need = pqkv_prefill_workspace_bytes(B, Hq, Hkv, Sq, S, d);
   if (!workspace || workspace_bytes < need)
     return fail(PQKV_ERR_WORKSPACE, "prefill: workspace %zu < %zu bytes", workspace_bytes, need);
-  const int64_t nvec = (int64_t)B * Hq * Sq;
-  const size_t arr = align256((size_t)nvec * d * 4);
+  // the faster plan if the workspace holds what it needs, else one workgroup
+  // per row block
+  pqkv::PrefillPlan plan = pqkv::prefill_plan(B, Hq, Hkv, Sq, S, d, qjl, true);
+  if (workspace_bytes < need + plan.bytes(d)) plan = pqkv::prefill_plan(B, Hq, Hkv, Sq, S, d, qjl, false);
+  float *part = (float *)((char *)workspace + need);
   float *q32 = (float *)workspace;
   float *o32 = (float *)((char *)workspace + arr);
   float *pq32 = (float *)((char *)workspace + 2 * arr);
@@ -963,7 +974,11 @@ int prefill_attn_run(const void *q, int q_dtype, const float *R, const uint8_t *
   a.S_max = S_max;
   a.d = d;
   a.causal = causal ? 1 : 0;
-  a.qt = pqkv::prefill_rows_per_block(qjl) / a.G;
+  a.qt = plan.qt;
+  a.qtiles = plan.qtiles;
+  a.splits = plan.splits;
+  a.part_o = part;
+  a.part_ml = part + plan.part_rows * d;
   if (pg) {
     a.k_pages = pg->k_pages;
     a.v_pages = pg->v_pages;

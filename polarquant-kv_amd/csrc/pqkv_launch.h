@@ -111,6 +111,8 @@ struct PrefillArgs {
   int B, Hq, Hkv, G, Sq, q_start, S, S_max, d, causal;
   int qt;                        // query tokens per workgroup (rows / G)
   int n_heads, listed;
+  int qtiles, splits;            // row blocks per stream; workgroups per row block
+  float *part_o, *part_ml;       // splits > 1: [stream][row block][row][split] (d floats; maximum and sum)
   // Paged caches (k_pages != null; k_cache / v_cache / qjl unused), as in
   // DecodeArgs: a 64-token tile lies in one page.
   const uint8_t *const *k_pages, *const *v_pages, *const *s_pages;
@@ -317,6 +319,19 @@ int device_compute_units();
 // Measurement: read `bytes` (a multiple of 16) from p once, XOR into sink[block].
 hipError_t launch_stream_read(const void *p, size_t bytes, uint32_t *sink, int blocks, hipStream_t s);
 hipError_t launch_prefill(const PrefillArgs &a, int k_bits, int v_bits, hipStream_t s);
+// How a prefill call runs: row blocks of `rows` query rows (qt tokens x G
+// heads), qtiles per (batch, kv-head) stream; splits > 1: each row block's
+// tokens over that many workgroups, their partials, in workspace beyond the
+// base (bytes(d)), joined by a merge launch. extra: whether there is such
+// workspace.
+struct PrefillPlan {
+  int rows, qt, qtiles, streams, splits;
+  int64_t part_rows;
+  size_t bytes(int d) const { return ((size_t)part_rows * (d + 2) * 4 + 255) & ~(size_t)255; }
+};
+PrefillPlan prefill_plan(int B, int Hq, int Hkv, int Sq, int S, int d, bool qjl, bool extra);
+// Joins a split launch's partials into a.o (streams stream0 .. + ns - 1).
+hipError_t launch_prefill_merge(const PrefillArgs &a, int stream0, int ns, int rows, hipStream_t s);
 // Query rows per prefill workgroup (the QJL kernel holds 16 rows per wave
 // instead of 32, to make room for the projection operands).
 int prefill_rows_per_block(bool qjl);

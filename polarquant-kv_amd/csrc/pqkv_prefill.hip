@@ -17,6 +17,10 @@
 // The waves run a two-group ping-pong schedule (matrix stage against softmax
 // and decode stage, one group a stage behind the other), described at the
 // main loop.
+// Workgroups: streams fastest, the longest row blocks first (causal prompts end
+// a launch on short ones). With splits > 1 a workgroup takes its share of the
+// row block's tiles and writes an unnormalised partial; prefill_merge_kernel
+// joins them.
 //
 // Scores are computed transposed, S^T[token][row] = K^ . Q^T: K^ (16 tokens x
 // 32 coordinates) is the A operand and the rotated queries the B operand, so
@@ -295,8 +299,11 @@ __global__ void __launch_bounds__(kPW * 64, 1) prefill_mfma_kernel(const Prefill
   const int gtid = tid - group * (kPW / 2) * 64;
   const int gw = __builtin_amdgcn_readfirstlane(wave) - group * (kPW / 2);
   const int G = a.G;
-  const int qtile = blockIdx.x;
-  const int bh = blockIdx.y;
+  // streams fastest, the longest row blocks (the last ones, with a causal
+  // mask) first
+  const int ns = a.B * a.n_heads, splits = a.splits;
+  const int bh = (int)blockIdx.x % ns, rest = (int)blockIdx.x / ns;
+  const int sp = rest % splits, qtile = a.qtiles - 1 - rest / splits;
   const int b = bh / a.n_heads, hl = bh - b * a.n_heads;
   const int h = a.listed ? a.heads[hl] : hl;
   const int q0 = qtile * a.qt;                       // first query token of the block
@@ -524,9 +531,10 @@ __global__ void __launch_bounds__(kPW * 64, 1) prefill_mfma_kernel(const Prefill
 #pragma unroll
         for (int i = 0; i < 4; ++i) cmax = fmaxf(cmax, s[tt][i]);
       cmax = rows_max(cmax);
-      // token 0 is valid for every row, so m_run is finite after the first tile
       const float mnew = fmaxf(m_run[rt], cmax);
-      const float alpha = __builtin_amdgcn_exp2f(m_run[rt] - mnew);
+      // a row with no visible token so far (splits) keeps weight 0
+      const float ref = mnew == -INFINITY ? 0.0f : mnew;
+      const float alpha = __builtin_amdgcn_exp2f(m_run[rt] - ref);
       m_run[rt] = mnew;
       float psum = 0.0f;
 #pragma unroll
@@ -535,7 +543,7 @@ __global__ void __launch_bounds__(kPW * 64, 1) prefill_mfma_kernel(const Prefill
         const float rr[4] = {r4.x, r4.y, r4.z, r4.w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float p = __builtin_amdgcn_exp2f(s[tt][i] - mnew);
+          const float p = __builtin_amdgcn_exp2f(s[tt][i] - ref);
           psum += p;
           half_t vh, vl;
           split2(p * rr[i], &vh, &vl);
@@ -572,7 +580,9 @@ __global__ void __launch_bounds__(kPW * 64, 1) prefill_mfma_kernel(const Prefill
   // 2 it - 1); group 1 decodes V(it + 1) in its Y(it) (stage 2 it + 2), after
   // group 1's values of tile it - 1 (stage 2 it + 1). Each is read from the
   // stage after its decode on, and radii follow their half.
-  const int ntiles = (kv_end + kPT - 1) / kPT;
+  // this workgroup's tiles: all of the row block's, or its split's share
+  const int all = (kv_end + kPT - 1) / kPT;
+  const int it0 = (int)((int64_t)all * sp / splits), it1 = (int)((int64_t)all * (sp + 1) / splits);
   uint8_t(&graw)[2][RawTile<D>::kAlloc] = raw[group];
   // The buffer tile t0 is copied from and t0's position in it: the whole
   // stream, or with paged caches (pages != null, a wave-uniform test) the
@@ -611,47 +621,47 @@ __global__ void __launch_bounds__(kPW * 64, 1) prefill_mfma_kernel(const Prefill
   // Block barrier for LDS hand-offs only: __syncthreads' release fence would
   // also wait for the raw-tile copies still in flight.
   auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-  if (ntiles > 0) dma(0);
-  if (ntiles > 1) dma(1);
+  if (it0 < it1) dma(it0);
+  if (it0 + 1 < it1) dma(it0 + 1);
   wait_dma();
   __syncthreads();  // tables and the first two raw tiles ready
-  if (ntiles > 0) decode(0);
-  __syncthreads();  // tile 0 decoded
+  if (it0 < it1) decode(it0);
+  __syncthreads();  // the first tile decoded
 
   // One loop per group (the compiler then sees that the scores and the
-  // weights are never live together); both make 2 ntiles + 2 barrier calls.
+  // weights are never live together); both make the same number of barriers.
   // Raw tile it + 2 streams into LDS from Y(it) on (after tile it + 1's
   // decode freed nothing it needs: it overwrites tile it's raw buffer); each
   // wave waits for its copies before the barrier that ends its next X stage.
   auto x_stage = [&](int it) {
     __builtin_amdgcn_s_setprio(1);
-    if (it >= 1) values(it - 1);
+    if (it > it0) values(it - 1);
     __builtin_amdgcn_sched_barrier(0);  // weights die before the scores start
-    if (it < ntiles) scores(it);
+    if (it < it1) scores(it);
     __builtin_amdgcn_s_setprio(0);
     wait_dma();
   };
   auto y_stage = [&](int it) {
     softmax(it);
-    if (it + 1 < ntiles) {
+    if (it + 1 < it1) {
       decode(it + 1);
-      if (it + 2 < ntiles) dma(it + 2);
+      if (it + 2 < it1) dma(it + 2);
     }
   };
-  if (ntiles > 0) {
+  if (it0 < it1) {
     if (group == 0) {
-      for (int it = 0; it <= ntiles; ++it) {
+      for (int it = it0; it <= it1; ++it) {
         x_stage(it);                                   // stage 2 it
         barrier();
-        if (it < ntiles) y_stage(it);                  // stage 2 it + 1
+        if (it < it1) y_stage(it);                     // stage 2 it + 1
         barrier();
       }
     } else {
       barrier();                                 // stage 0
-      for (int it = 0; it <= ntiles; ++it) {
+      for (int it = it0; it <= it1; ++it) {
         x_stage(it);                                   // stage 2 it + 1
         barrier();
-        if (it < ntiles) {                             // stage 2 it + 2
+        if (it < it1) {                                // stage 2 it + 2
           y_stage(it);
           barrier();
         }
@@ -659,24 +669,56 @@ __global__ void __launch_bounds__(kPW * 64, 1) prefill_mfma_kernel(const Prefill
     }
   }
 
-  // ---------------- normalise and write o_rot ----------------
+  // ---------------- normalise and write o_rot, or the split's partial ----------------
+  const int64_t prow0 = ((int64_t)bh * a.qtiles + qtile) * (16 * RT * kPW);
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     const float l = rows_sum(l_run[rt]);
+    if (splits > 1 && grp == 0)
+      ((float2 *)a.part_ml)[(prow0 + 16 * RT * wave + 16 * rt + col) * splits + sp] = make_float2(m_run[rt], l);
     float f[4];
-    per_row(l > 0.0f ? 1.0f / (l * kPlaneScale) : 0.0f, grp, f);   // the value planes' 2^6 as well
+    per_row(splits > 1 ? 1.0f : l > 0.0f ? 1.0f / (l * kPlaneScale) : 0.0f, grp, f);   // the value planes' 2^6 as well
     // output rows 4 grp + i of this row tile
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int row = 16 * RT * wave + 16 * rt + 4 * grp + i;
       const int tok = q0 + row / G, head = row % G;
-      if (row < a.qt * G && tok < a.Sq) {
-        float *dst = a.o + (((int64_t)(b * a.Hq + h * G + head) * a.Sq) + tok) * D;
+      float *dst;
+      if (splits > 1) dst = a.part_o + ((prow0 + row) * splits + sp) * D;
+      else if (row < a.qt * G && tok < a.Sq) dst = a.o + (((int64_t)(b * a.Hq + h * G + head) * a.Sq) + tok) * D;
+      else continue;
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) dst[16 * nb + col] = oacc[rt][nb][i] * f[i];
-      }
+      for (int nb = 0; nb < NB; ++nb) dst[16 * nb + col] = oacc[rt][nb][i] * f[i];
     }
   }
+}
+
+// Joins the splits of each query row: o = sum_s 2^(m_s - m) o_s / sum_s 2^(m_s
+// - m) l_s. D / 4 threads per row.
+template <int D>
+__global__ void __launch_bounds__(256) prefill_merge_kernel(const PrefillArgs a, int stream0, int rows) {
+  constexpr int TR = D / 4, RB = 256 / TR;
+  const int sl = blockIdx.y, bh = stream0 + sl, splits = a.splits;
+  const int b = bh / a.n_heads, hl = bh - b * a.n_heads;
+  const int h = a.listed ? a.heads[hl] : hl;
+  const int64_t at = (int64_t)blockIdx.x * RB + threadIdx.x / TR;   // row of the stream's padded rows
+  const int qtile = (int)(at / rows), rw = (int)(at % rows);
+  const int tk = qtile * a.qt + rw / a.G;
+  if (qtile >= a.qtiles || rw >= a.qt * a.G || tk >= a.Sq) return;
+  const int64_t prow = (int64_t)sl * a.qtiles * rows + at;
+  const float2 *ml = (const float2 *)a.part_ml + prow * splits;
+  float m = -INFINITY;
+  for (int s = 0; s < splits; ++s) m = fmaxf(m, ml[s].x);
+  float L = 0.0f;
+  float4_t o = {0.f, 0.f, 0.f, 0.f};
+  const float4_t *po = (const float4_t *)(a.part_o + prow * splits * D) + threadIdx.x % TR;
+  for (int s = 0; s < splits; ++s) {
+    const float w = ml[s].x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml[s].x - m);
+    L += w * ml[s].y;
+    o += w * po[(int64_t)s * TR];
+  }
+  const float inv = L > 0.0f ? 1.0f / (L * kPlaneScale) : 0.0f;
+  *((float4_t *)(a.o + ((int64_t)(b * a.Hq + h * a.G + rw % a.G) * a.Sq + tk) * D) + threadIdx.x % TR) = o * inv;
 }
 
 template <int D, int KB, int VBITS>
@@ -693,12 +735,48 @@ static void launch_pd(const PrefillArgs &a, int kb, int vb, dim3 grid, hipStream
   else launch_pw<D, 2, 2>(a, grid, s);
 }
 
+// Few row blocks: one round of workgroups (one per compute unit) leaves
+// compute units idle, so each block's tokens are split over several. Measured
+// (fp32 out, d = 128, 32 query / 8 kv heads, batch 1, launch before / after
+// with the rotations on the matrix cores): 16 query tokens against 65 000
+// cached 4348 -> 177 us, 512 against 3584 348 -> 126 us.
+constexpr int kTargetBlocks = 256;
+
+PrefillPlan prefill_plan(int B, int Hq, int Hkv, int Sq, int S, int d, bool qjl, bool extra) {
+  PrefillPlan p{};
+  const int G = Hq / Hkv;
+  p.rows = prefill_rows_per_block(qjl);
+  p.qt = p.rows / G;
+  p.qtiles = (Sq + p.qt - 1) / p.qt;
+  p.splits = 1;
+  p.streams = B * Hkv;
+  if (!extra || S < 1) return p;
+  const int tiles = (S + kPT - 1) / kPT;
+  const int64_t blocks = (int64_t)p.qtiles * p.streams;
+  int64_t splits = kTargetBlocks / blocks;
+  if (splits > tiles / 4) splits = tiles / 4;   // a split of four tiles at least
+  if (splits > 1) {
+    p.splits = (int)splits;
+    p.part_rows = blocks * p.rows * splits;
+  }
+  return p;
+}
+
+hipError_t launch_prefill_merge(const PrefillArgs &a, int stream0, int ns, int rows, hipStream_t s) {
+  const int rb = 256 / (a.d / 4);
+  const dim3 grid((a.qtiles * rows + rb - 1) / rb, ns);
+  if (a.d == 128) prefill_merge_kernel<128><<<grid, 256, 0, s>>>(a, stream0, rows);
+  else prefill_merge_kernel<64><<<grid, 256, 0, s>>>(a, stream0, rows);
+  return hipGetLastError();
+}
+
 hipError_t launch_prefill(const PrefillArgs &a, int k_bits, int v_bits, hipStream_t s) {
-  const int qtiles = (a.Sq + a.qt - 1) / a.qt;
-  dim3 grid(qtiles, a.B * a.n_heads);
+  const dim3 grid(a.qtiles * a.splits * a.B * a.n_heads);
   if (a.d == 128) launch_pd<128>(a, k_bits, v_bits, grid, s);
   else launch_pd<64>(a, k_bits, v_bits, grid, s);
-  return hipGetLastError();
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || a.splits == 1) return e;
+  return launch_prefill_merge(a, 0, a.B * a.n_heads, prefill_rows_per_block(a.qjl != nullptr || a.s_pages != nullptr), s);
 }
 
 int prefill_rows_per_block(bool qjl) { return kPW * (qjl ? kPRowsWave / 2 : kPRowsWave); }

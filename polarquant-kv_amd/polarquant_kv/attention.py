@@ -211,7 +211,7 @@ def prefill_attention(query: torch.Tensor, keys: PQCache, values: PQCache, rotat
     out = torch.empty(B, Hq, Sq, d, dtype=out_dtype, device=q.device)
     lib = _lib.lib()
     S = keys.seq_len
-    need = lib.pqkv_prefill_workspace_bytes(B, Hq, Hkv, Sq, max(S, 1), d)
+    need = lib.pqkv_prefill_workspace_preferred_bytes(B, Hq, Hkv, Sq, max(S, 1), d, int(jl_rot is not None))
     ws = torch.empty(max(need, 1), dtype=torch.uint8, device=q.device)
     mixed = keys.mixed or values.mixed
     kbits = _lib.int_array(keys.head_bits()) if mixed else None
@@ -241,7 +241,7 @@ def _prefill_paged(query, keys, values, rotation_matrix, q_start, causal, scale,
     out = torch.empty(B, Hq, Sq, d, dtype=out_dtype, device=q.device)
     lib = _lib.lib()
     S = keys.seq_len
-    need = lib.pqkv_prefill_workspace_bytes(B, Hq, Hkv, Sq, max(S, 1), d)
+    need = lib.pqkv_prefill_workspace_preferred_bytes(B, Hq, Hkv, Sq, max(S, 1), d, int(jl_rot is not None))
     ws = torch.empty(max(need, 1), dtype=torch.uint8, device=q.device)
     if jl_rot is not None and keys.sign_table is None:
         raise ValueError("QJL correction requested but the key cache has no signs")
