@@ -341,8 +341,9 @@ int pqkv_soa_attn_generic(const float *q_rot, const uint8_t *k_codes, const floa
  * pqkv_decode_attn. */
 size_t pqkv_prefill_workspace_bytes(int B, int Hq, int Hkv, int Sq, int S, int d);
 /* The workspace with which pqkv_prefill_attn (and _paged) is fastest: at least
- * pqkv_prefill_workspace_bytes, with room to split the tokens of small calls
- * over more workgroups. Any size from the smaller one on is accepted. */
+ * pqkv_prefill_workspace_bytes; for long chunks (without QJL) also room for
+ * the cache's tiles decoded once per call, about 1 KB per cached token and kv
+ * head at d = 128, at most 2 GiB. Any size from the smaller one on is accepted. */
 size_t pqkv_prefill_workspace_preferred_bytes(int B, int Hq, int Hkv, int Sq, int S, int d, int qjl);
 
 int pqkv_prefill_attn(const void *q, int q_dtype, const float *R,

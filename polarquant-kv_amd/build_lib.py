@@ -24,7 +24,7 @@ SOURCES = ["pqkv_encode.hip", "pqkv_rotate_mfma.hip", "pqkv_encode_chain.hip", "
            "pqkv_decode_mfma_k4v4_shared.hip", "pqkv_decode_mfma_k4v4_own.hip", "pqkv_decode_mfma_k4v2.hip",
            "pqkv_decode_mfma_k2v4.hip", "pqkv_decode_mfma_k2v2.hip", "pqkv_decode_mfma_pair.hip",
            "pqkv_decode_mfma_soa.hip", "pqkv_decode_mfma_paged_k4v4_shared.hip", "pqkv_decode_mfma_paged_k4v4_own.hip",
-           "pqkv_decode_mfma_paged_k2v2.hip", "pqkv_decode_mfma_ggml.hip", "pqkv_prefill.hip", "pqkv_group.hip", "pqkv_group_gpu.hip", "pqkv_group_mfma.hip", "pqkv_group_api.cpp",
+           "pqkv_decode_mfma_paged_k2v2.hip", "pqkv_decode_mfma_ggml.hip", "pqkv_prefill.hip", "pqkv_prefill_planes.hip", "pqkv_group.hip", "pqkv_group_gpu.hip", "pqkv_group_mfma.hip", "pqkv_group_api.cpp",
            "pqkv_api.cpp", "pqkv_compat.cpp", "pqkv_ggml.cpp", "pqkv_noalloc.hip"]
 
 

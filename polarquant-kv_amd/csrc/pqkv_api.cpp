@@ -937,10 +937,11 @@ int prefill_attn_run(const void *q, int q_dtype, const float *R, const uint8_t *
   if (!workspace || workspace_bytes < need)
     return fail(PQKV_ERR_WORKSPACE, "prefill: workspace %zu < %zu bytes", workspace_bytes, need);
   // the faster plan if the workspace holds what it needs, else one workgroup
-  // per row block
+  // per row block that decodes the tiles itself
   pqkv::PrefillPlan plan = pqkv::prefill_plan(B, Hq, Hkv, Sq, S, d, qjl, true);
   if (workspace_bytes < need + plan.bytes(d)) plan = pqkv::prefill_plan(B, Hq, Hkv, Sq, S, d, qjl, false);
   float *part = (float *)((char *)workspace + need);
+  uint8_t *records = (uint8_t *)part + plan.part_bytes(d);
   float *q32 = (float *)workspace;
   float *o32 = (float *)((char *)workspace + arr);
   float *pq32 = (float *)((char *)workspace + 2 * arr);
@@ -992,10 +993,13 @@ int prefill_attn_run(const void *q, int q_dtype, const float *R, const uint8_t *
     a.k_batch_stride = a.k_head_stride * Hkv;
     a.v_batch_stride = a.v_head_stride * Hkv;
     a.n_heads = Hkv;
+    a.k_tok_stride = pqkv_vector_bytes(d, k_bits);
+    a.v_tok_stride = pqkv_vector_bytes(d, v_bits);
     tok = pqkv::prof_begin("prefill_attn", st, true);
     e = hipSuccess;
     for (int rep = 0, nrep = pqkv::prof_repeats(); rep < nrep && e == hipSuccess; ++rep)
-      e = pqkv::launch_prefill(a, k_bits, v_bits, st);
+      e = plan.planes ? pqkv::launch_prefill_planes(a, k_bits, v_bits, plan, records, st)
+                      : pqkv::launch_prefill(a, k_bits, v_bits, st);
     pqkv::prof_end(tok, st);
     if (e != hipSuccess) return hip_status(e, "prefill launch");
   } else {
@@ -1022,10 +1026,13 @@ int prefill_attn_run(const void *q, int q_dtype, const float *R, const uint8_t *
           }
         if (n == 0) continue;
         a.n_heads = n;
+        a.k_tok_stride = pqkv_vector_bytes(d, kbits);
+        a.v_tok_stride = pqkv_vector_bytes(d, vbits);
         tok = pqkv::prof_begin("prefill_attn", st, true);
         e = hipSuccess;
         for (int rep = 0, nrep = pqkv::prof_repeats(); rep < nrep && e == hipSuccess; ++rep)
-          e = pqkv::launch_prefill(a, kbits, vbits, st);
+          e = plan.planes ? pqkv::launch_prefill_planes(a, kbits, vbits, plan, records, st)
+                          : pqkv::launch_prefill(a, kbits, vbits, st);
         pqkv::prof_end(tok, st);
         if (e != hipSuccess) return hip_status(e, "prefill launch");
       }

@@ -111,6 +111,7 @@ struct PrefillArgs {
   int B, Hq, Hkv, G, Sq, q_start, S, S_max, d, causal;
   int qt;                        // query tokens per workgroup (rows / G)
   int n_heads, listed;
+  int64_t k_tok_stride, v_tok_stride;   // bytes between tokens (pre-decoded tiles only)
   int qtiles, splits;            // row blocks per stream; workgroups per row block
   float *part_o, *part_ml;       // splits > 1: [stream][row block][row][split] (d floats; maximum and sum)
   // Paged caches (k_pages != null; k_cache / v_cache / qjl unused), as in
@@ -320,16 +321,22 @@ int device_compute_units();
 hipError_t launch_stream_read(const void *p, size_t bytes, uint32_t *sink, int blocks, hipStream_t s);
 hipError_t launch_prefill(const PrefillArgs &a, int k_bits, int v_bits, hipStream_t s);
 // How a prefill call runs: row blocks of `rows` query rows (qt tokens x G
-// heads), qtiles per (batch, kv-head) stream; splits > 1: each row block's
-// tokens over that many workgroups, their partials, in workspace beyond the
-// base (bytes(d)), joined by a merge launch. extra: whether there is such
-// workspace.
+// heads), qtiles per (batch, kv-head) stream; planes: over tiles decoded once
+// per call (pqkv_prefill_planes.hip), `streams` streams at a time, else by the
+// kernel that decodes them per row block; splits > 1: each row block's tokens
+// over that many workgroups, their partials joined by a merge launch. Both
+// need workspace beyond the base: bytes(d) = the partials, then the records.
 struct PrefillPlan {
+  bool planes;
   int rows, qt, qtiles, streams, splits;
-  int64_t part_rows;
-  size_t bytes(int d) const { return ((size_t)part_rows * (d + 2) * 4 + 255) & ~(size_t)255; }
+  int64_t stream_bytes, part_rows;
+  size_t part_bytes(int d) const { return ((size_t)part_rows * (d + 2) * 4 + 255) & ~(size_t)255; }
+  size_t bytes(int d) const { return part_bytes(d) + (planes ? (size_t)streams * stream_bytes : 0); }
 };
+inline int64_t prefill_record_bytes(int d) { return 512 * (int64_t)d + 512; }   // one decoded 64-token tile
 PrefillPlan prefill_plan(int B, int Hq, int Hkv, int Sq, int S, int d, bool qjl, bool extra);
+hipError_t launch_prefill_planes(PrefillArgs a, int k_bits, int v_bits, const PrefillPlan &p, uint8_t *records,
+                                 hipStream_t s);
 // Joins a split launch's partials into a.o (streams stream0 .. + ns - 1).
 hipError_t launch_prefill_merge(const PrefillArgs &a, int stream0, int ns, int rows, hipStream_t s);
 // Query rows per prefill workgroup (the QJL kernel holds 16 rows per wave

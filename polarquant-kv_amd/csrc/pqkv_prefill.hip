@@ -741,6 +741,7 @@ static void launch_pd(const PrefillArgs &a, int kb, int vb, dim3 grid, hipStream
 // with the rotations on the matrix cores): 16 query tokens against 65 000
 // cached 4348 -> 177 us, 512 against 3584 348 -> 126 us.
 constexpr int kTargetBlocks = 256;
+constexpr int64_t kPlaneBudget = (int64_t)2 << 30;   // bytes of decoded tiles at a time
 
 PrefillPlan prefill_plan(int B, int Hq, int Hkv, int Sq, int S, int d, bool qjl, bool extra) {
   PrefillPlan p{};
@@ -752,6 +753,20 @@ PrefillPlan prefill_plan(int B, int Hq, int Hkv, int Sq, int S, int d, bool qjl,
   p.streams = B * Hkv;
   if (!extra || S < 1) return p;
   const int tiles = (S + kPT - 1) / kPT;
+  // Decoding each tile once per call instead of once per row block pays from
+  // some row blocks on (records are written and read back, 1 KB per token at
+  // d = 128). Whole calls, decoded once / per row block: d = 128 12 row blocks
+  // 103 / 117 us, 24 181 / 194 us, 64 against 131 072 tokens 16.9 / 18.7 ms, but
+  // 8 2.66 / 2.34 ms (256 streams) and 2.03 / 1.83 ms (256), 117 / 126 us (8
+  // streams); d = 64 6 387 / 454 us, 8 3.47 / 3.55 ms, 28 76 / 86 us, but 1
+  // 326 / 244 us.
+  p.stream_bytes = (int64_t)tiles * prefill_record_bytes(d);
+  p.planes = !qjl && p.qtiles >= (d == 128 ? 12 : 6) && p.stream_bytes <= kPlaneBudget;
+  if (p.planes) {
+    // equal passes over the streams
+    const int64_t all = p.streams, fit = kPlaneBudget / p.stream_bytes, passes = (all + fit - 1) / fit;
+    p.streams = (int)((all + passes - 1) / passes);
+  }
   const int64_t blocks = (int64_t)p.qtiles * p.streams;
   int64_t splits = kTargetBlocks / blocks;
   if (splits > tiles / 4) splits = tiles / 4;   // a split of four tiles at least

@@ -1,5 +1,6 @@
-"""Chunked prefill with the preferred workspace (tokens split over workgroups)
-against the same call with the smallest one (a workgroup per row block): odd
+"""Chunked prefill with the preferred workspace (tokens split over workgroups;
+from 12 row blocks, 6 at d = 64, tiles decoded once per call) against the same
+call with the smallest one (a workgroup per row block that decodes them): odd
 lengths, chunks whose early rows see none of a split's tokens, sign corrections,
 per-head widths, paged caches."""
 
@@ -15,7 +16,8 @@ DEV = "cuda:0"
 
 # (B, Hq, Hkv, Sq, q_start, d, causal)
 SHAPES = [(1, 8, 2, 9, 1000, 128, 1), (2, 14, 2, 33, 2111, 64, 1), (1, 4, 1, 300, 515, 128, 1),
-          (1, 32, 8, 130, 4000, 128, 0), (3, 6, 2, 65, 767, 64, 0), (1, 1, 1, 513, 0, 128, 1)]
+          (1, 32, 8, 130, 4000, 128, 0), (3, 6, 2, 65, 767, 64, 0), (1, 1, 1, 513, 0, 128, 1),
+          (1, 8, 2, 801, 100, 128, 1), (2, 14, 2, 300, 1003, 64, 1), (1, 4, 4, 3073, 0, 128, 1), (1, 14, 2, 217, 333, 64, 0)]
 
 
 def _run(q, kc, vc, R, jl, q_start, causal, preferred):
