@@ -68,7 +68,11 @@ typedef __attribute__((address_space(3))) const u32x2 lds_cu32x2;
 __device__ __forceinline__ void lds_put8(uint8_t *p, uint32_t a, uint32_t b) { *(lds_u32x2 *)p = (u32x2){a, b}; }
 __device__ __forceinline__ u32x2 lds_get8(const uint8_t *p) { return *(lds_cu32x2 *)p; }
 
+// x is made opaque first: otherwise the compiler rounds a product once for lo's
+// hi (v_fma_mixlo_f16) and twice for the stored one, and where they differ the
+// pair is off by an fp16 step (1e-3 of a weight, in one of some thousands).
 __device__ __forceinline__ void split2(float x, half_t *hi, half_t *lo) {
+  asm("" : "+v"(x));
   const half_t h = (half_t)x;
   *hi = h;
   *lo = (half_t)(x - (float)h);

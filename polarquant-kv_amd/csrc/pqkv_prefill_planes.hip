@@ -72,7 +72,11 @@ struct PlaneRec {
   __host__ __device__ static constexpr int vseg(int nb, int kk, int plane) { return (nb * 2 + kk) * 2 + plane; }
 };
 
+// x is made opaque first: otherwise the compiler rounds a product once for lo's
+// hi (v_fma_mixlo_f16) and twice for the stored one, and where they differ the
+// pair is off by an fp16 step (1e-3 of a weight, in one of some thousands).
 __device__ __forceinline__ void split2(float x, half_t *hi, half_t *lo) {
+  asm("" : "+v"(x));
   const half_t h = (half_t)x;
   *hi = h;
   *lo = (half_t)(x - (float)h);
