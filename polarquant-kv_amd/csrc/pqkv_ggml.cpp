@@ -256,11 +256,27 @@ int pqkv_ggml_cpy_pq4(const polarquant_state *st, const void *src, int src_type,
 
 namespace {
 
+// From these query rows per sequence and this work (query rows x kv heads x
+// tokens x d) on, the cache is decoded once per call instead of streamed once
+// per row. Whole calls, streamed / decoded once, us: 32 query / 8 kv heads, d =
+// 128, 64 rows against 4096 tokens (2^28) 75 / 69, 512 against 512 (2^28) 150 /
+// 71, but 2 x 16 against 4096 (2^27) 46 / 74; 32 / 32 heads 64 against 4096 207
+// / 104, but 2 x 16 (2^29) 115 / 187, 64 against 512 (2^27) 48 / 56; 64 / 8
+// heads 64 against 4096 102 / 75; d = 64, 14 / 2 heads, 512 against 4096 (2^28)
+// 116 / 68, against 512 39 / 42.
+constexpr int kManyRows = 64;
+constexpr int64_t kManyWork = (int64_t)1 << 28;
+
 // The validated shape of one flash_attn_ext call.
 struct FaShape {
   int d, n_q, Hq, n_seq, n_kv, Hkv;
   int splits, tps;
   size_t q_off, part_off, bytes;
+  // several query rows per sequence: the prefill kernel over tiles decoded
+  // once per call, where the caller's workspace has room for it
+  bool many;
+  pqkv::PrefillPlan plan;
+  size_t o_off, extra_off, many_bytes;
 };
 
 int fa_shape(const polarquant_state *st, const int64_t ne_q[4], const int64_t ne_k[4], FaShape *f) {
@@ -297,6 +313,18 @@ int fa_shape(const polarquant_state *st, const int64_t ne_q[4], const int64_t ne
   if (rows > 0 && f->n_kv > 0) pqkv::mfma_split_plan(wg_rows, f->n_kv, &f->splits, &f->tps);
   size_t pq_off;
   f->bytes = pqkv::decode_workspace_layout((int)rows, f->Hq, f->splits, d, &f->q_off, &f->part_off, &pq_off);
+  f->many = false;
+  f->many_bytes = f->bytes;
+  if (f->n_seq > 0 && f->n_q >= kManyRows && f->Hq > 0 && f->n_kv > 0 && f->n_kv % 4 == 0 &&
+      (double)rows * f->Hkv * f->n_kv * d >= (double)kManyWork &&
+      f->Hq / f->Hkv <= pqkv::prefill_rows_per_block(false)) {
+    f->plan = pqkv::prefill_plan(f->n_seq, f->Hq, f->Hkv, f->n_q, f->n_kv, d, false, true, true);
+    f->many = f->plan.planes;
+    const size_t arr = ((size_t)rows * f->Hq * d * 4 + 255) & ~(size_t)255;
+    f->o_off = arr;                              // queries, output, partials and records
+    f->extra_off = 2 * arr;
+    if (f->many) f->many_bytes = std::max(f->bytes, 2 * arr + f->plan.bytes(d));
+  }
   return PQKV_OK;
 }
 
@@ -307,7 +335,7 @@ extern "C" {
 size_t pqkv_ggml_flash_attn_ext_pq4_workspace_bytes(const polarquant_state *st, const int64_t ne_q[4],
                                                     const int64_t ne_k[4]) {
   FaShape f;
-  return fa_shape(st, ne_q, ne_k, &f) == PQKV_OK ? f.bytes : 0;
+  return fa_shape(st, ne_q, ne_k, &f) == PQKV_OK ? f.many_bytes : 0;
 }
 
 int pqkv_ggml_flash_attn_ext_pq4(const polarquant_state *st, const float *q, const int64_t ne_q[4],
@@ -361,14 +389,60 @@ int pqkv_ggml_flash_attn_ext_pq4(const polarquant_state *st, const float *q, con
   if (!workspace || workspace_bytes < f.bytes)
     return pqkv::fail_status(PQKV_ERR_WORKSPACE, "ggml flash_attn_ext: workspace %zu < %zu bytes", workspace_bytes,
                              f.bytes);
-  float *q32 = (float *)((char *)workspace + f.q_off);
-  float *part = (float *)((char *)workspace + f.part_off);
+  // the mask as the prefill kernel reads it: four tokens' values at a time
+  const bool many = f.many && workspace_bytes >= f.many_bytes && (uintptr_t)workspace % 16 == 0 &&
+                    (uintptr_t)mask % 8 == 0 && m_row % 4 == 0 && m_seq % 4 == 0;
+  float *q32 = (float *)((char *)workspace + (many ? 0 : f.q_off));
+  float *part = (float *)((char *)workspace + (many ? f.extra_off : f.part_off));
   const float kLog2e = 1.4426950408889634f;
   int tok = pqkv::prof_begin("ggml_fa_rotate", s);
   hipError_t e = pqkv::launch_rotate_rows(q, (int64_t)(nb_q[1] / 4), (int64_t)(nb_q[2] / 4), (int64_t)(nb_q[3] / 4),
                                           f.n_q, f.Hq, f.n_seq, st->rotation, q32, f.d, scale * kLog2e, s);
   pqkv::prof_end(tok, s);
   if (e != hipSuccess) return pqkv::report_hip_error(e, "ggml flash_attn_ext query rotation");
+
+  if (many) {
+    float *o32 = (float *)((char *)workspace + f.o_off);
+    pqkv::PrefillArgs p;
+    std::memset(&p, 0, sizeof(p));
+    p.q = q32;
+    p.k_cache = (const uint8_t *)k;
+    p.v_cache = (const uint8_t *)v;
+    p.k_cb = p.v_cb = st->codebook;
+    p.o = o32;
+    p.B = f.n_seq;
+    p.Hq = f.Hq;
+    p.Hkv = p.n_heads = f.Hkv;
+    p.G = f.Hq / f.Hkv;
+    p.Sq = f.n_q;
+    p.S = p.S_max = f.n_kv;
+    p.d = f.d;
+    p.qt = f.plan.qt;
+    p.qtiles = f.plan.qtiles;
+    p.splits = f.plan.splits;
+    p.part_o = part;
+    p.part_ml = part + f.plan.part_rows * f.d;
+    p.k_tok_stride = (int64_t)nb_k[1];
+    p.v_tok_stride = (int64_t)nb_v[1];
+    p.k_head_stride = (int64_t)nb_k[2];
+    p.v_head_stride = (int64_t)nb_v[2];
+    p.k_batch_stride = ne_k[3] == 1 ? 0 : (int64_t)nb_k[3];
+    p.v_batch_stride = ne_v[3] == 1 ? 0 : (int64_t)nb_v[3];
+    p.token_major = 1;
+    p.mask = mrow;
+    p.mask_row_stride = m_row;
+    p.mask_seq_stride = m_seq;
+    tok = pqkv::prof_begin("ggml_fa_prefill", s, true);
+    e = hipSuccess;
+    for (int rep = 0, nrep = pqkv::prof_repeats(); rep < nrep && e == hipSuccess; ++rep)
+      e = pqkv::launch_prefill_planes(p, 4, 4, f.plan, (uint8_t *)part + f.plan.part_bytes(f.d), s);
+    pqkv::prof_end(tok, s);
+    if (e != hipSuccess) return pqkv::report_hip_error(e, "ggml flash_attn_ext prefill launch");
+    tok = pqkv::prof_begin("ggml_fa_rotate_out", s);
+    e = pqkv::launch_rotate(o32, PQKV_F32, st->rotation, dst, PQKV_F32, rows * f.Hq, f.d, 1, 1.0f, s);
+    pqkv::prof_end(tok, s);
+    return pqkv::report_hip_error(e, "ggml flash_attn_ext output rotation");
+  }
 
   pqkv::DecodeArgs a;
   std::memset(&a, 0, sizeof(a));

@@ -113,6 +113,12 @@ struct PrefillArgs {
   int n_heads, listed;
   int64_t k_tok_stride, v_tok_stride;   // bytes between tokens (pre-decoded tiles only)
   int qtiles, splits;            // row blocks per stream; workgroups per row block
+  // Pre-decoded tiles in llama.cpp's layout: q and o [B][Sq][Hq][d], q without
+  // kPrefillPlaneScale, S a multiple of 4, and an additive fp16 mask (or null)
+  // on an 8-byte boundary, strides in elements and multiples of 4.
+  int token_major;
+  const uint16_t *mask;
+  int64_t mask_row_stride, mask_seq_stride;
   float *part_o, *part_ml;       // splits > 1: [stream][row block][row][split] (d floats; maximum and sum)
   // Paged caches (k_pages != null; k_cache / v_cache / qjl unused), as in
   // DecodeArgs: a 64-token tile lies in one page.
@@ -334,7 +340,9 @@ struct PrefillPlan {
   size_t bytes(int d) const { return part_bytes(d) + (planes ? (size_t)streams * stream_bytes : 0); }
 };
 inline int64_t prefill_record_bytes(int d) { return 512 * (int64_t)d + 512; }   // one decoded 64-token tile
-PrefillPlan prefill_plan(int B, int Hq, int Hkv, int Sq, int S, int d, bool qjl, bool extra);
+// extra: the workspace holds what the plan asks for; planes_only: over tiles
+// decoded once, at any count of row blocks, where a stream's fit their budget.
+PrefillPlan prefill_plan(int B, int Hq, int Hkv, int Sq, int S, int d, bool qjl, bool extra, bool planes_only = false);
 hipError_t launch_prefill_planes(PrefillArgs a, int k_bits, int v_bits, const PrefillPlan &p, uint8_t *records,
                                  hipStream_t s);
 // Joins a split launch's partials into a.o (streams stream0 .. + ns - 1).

@@ -722,7 +722,9 @@ __global__ void __launch_bounds__(256) prefill_merge_kernel(const PrefillArgs a,
     o += w * po[(int64_t)s * TR];
   }
   const float inv = L > 0.0f ? 1.0f / (L * kPlaneScale) : 0.0f;
-  *((float4_t *)(a.o + ((int64_t)(b * a.Hq + h * a.G + rw % a.G) * a.Sq + tk) * D) + threadIdx.x % TR) = o * inv;
+  const int64_t head = h * a.G + rw % a.G;
+  const int64_t orow = a.token_major ? ((int64_t)b * a.Sq + tk) * a.Hq + head : (b * a.Hq + head) * a.Sq + tk;
+  *((float4_t *)(a.o + orow * D) + threadIdx.x % TR) = o * inv;
 }
 
 template <int D, int KB, int VBITS>
@@ -747,7 +749,7 @@ static void launch_pd(const PrefillArgs &a, int kb, int vb, dim3 grid, hipStream
 constexpr int kTargetBlocks = 256;
 constexpr int64_t kPlaneBudget = (int64_t)2 << 30;   // bytes of decoded tiles at a time
 
-PrefillPlan prefill_plan(int B, int Hq, int Hkv, int Sq, int S, int d, bool qjl, bool extra) {
+PrefillPlan prefill_plan(int B, int Hq, int Hkv, int Sq, int S, int d, bool qjl, bool extra, bool planes_only) {
   PrefillPlan p{};
   const int G = Hq / Hkv;
   p.rows = prefill_rows_per_block(qjl);
@@ -765,7 +767,7 @@ PrefillPlan prefill_plan(int B, int Hq, int Hkv, int Sq, int S, int d, bool qjl,
   // streams); d = 64 6 387 / 454 us, 8 3.47 / 3.55 ms, 28 76 / 86 us, but 1
   // 326 / 244 us.
   p.stream_bytes = (int64_t)tiles * prefill_record_bytes(d);
-  p.planes = !qjl && p.qtiles >= (d == 128 ? 12 : 6) && p.stream_bytes <= kPlaneBudget;
+  p.planes = !qjl && (planes_only || p.qtiles >= (d == 128 ? 12 : 6)) && p.stream_bytes <= kPlaneBudget;
   if (p.planes) {
     // equal passes over the streams
     const int64_t all = p.streams, fit = kPlaneBudget / p.stream_bytes, passes = (all + fit - 1) / fit;

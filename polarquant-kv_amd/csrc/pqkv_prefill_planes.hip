@@ -58,6 +58,7 @@ constexpr float kScoreUnscale = 1.0f / (kPlaneScale * kPlaneScale);
 
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(3))) const half8_t lds_chalf8;
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 template <int D>
 struct PlaneRec {
@@ -202,7 +203,11 @@ __global__ void __launch_bounds__(256) plane_decode_kernel(const PrefillArgs a, 
 }
 
 // ---------------------------------------------------------------------------
-template <int D>
+// GG (llama.cpp's flash_attn_ext): queries and output [sequence][token][head],
+// an additive fp16 mask in the place of the causal rule, and the operands'
+// powers of two follow the data (queries per row, weights times radii by the
+// largest value radius so far), since they are fp32 there and the results too.
+template <int D, bool GG>
 __global__ void __launch_bounds__(kPW * 64, 1)
     prefill_planes_kernel(const PrefillArgs a, const uint8_t *planes, int64_t stream_bytes, int stream0, int ns) {
   using P = PlaneRec<D>;
@@ -241,20 +246,39 @@ __global__ void __launch_bounds__(kPW * 64, 1)
   // col; step ks, slot k = 8 grp + i is coordinate 32 ks + 8 grp + i
   half8_t qh[RT][KS], ql[RT][KS];
   int row_pos[RT];
+  float q_un[RT];                              // GG: undoes the row's query scale (beside the radii's 2^-12)
+  const uint16_t *mrow[RT];                    // GG: the row's mask
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     const int row = 32 * wave + 16 * rt + col;
     const int tok = q0 + row / G, head = row % G;
     const bool row_ok = row < a.qt * G && tok < a.Sq;
     row_pos[rt] = a.q_start + tok;
-    const float *qr = a.q + ((int64_t)(b * a.Hq + h * G + head) * a.Sq + (row_ok ? tok : 0)) * D;
+    const int64_t qrow = GG ? ((int64_t)b * a.Sq + (row_ok ? tok : 0)) * a.Hq + h * G + head
+                            : (int64_t)(b * a.Hq + h * G + head) * a.Sq + (row_ok ? tok : 0);
+    const float *qr = a.q + qrow * D;
+    float q_sc = 1.0f;
+    if constexpr (GG) {
+      float amax = 0.0f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(qr[32 * ks + 8 * grp + i]));
+      // the row's largest value to [2^8, 2^9) (as it is if zero, subnormal or not finite)
+      const int ex = (int)(__builtin_bit_cast(uint32_t, rows_max(amax)) >> 23);
+      const int sh = ex == 0 || ex == 255 ? 0 : min(135 - ex, 100);
+      q_sc = __builtin_ldexpf(1.0f, sh);
+      q_un[rt] = __builtin_ldexpf(kPlaneScale, -sh);
+      mrow[rt] = a.mask + b * a.mask_seq_stride + (row_ok ? tok : 0) * a.mask_row_stride;
+    }
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const float4_t x0 = *(const float4_t *)(qr + 32 * ks + 8 * grp), x1 = *(const float4_t *)(qr + 32 * ks + 8 * grp + 4);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         half_t vh, vl;
-        split2(row_ok ? (i < 4 ? x0[i & 3] : x1[i & 3]) : 0.0f, &vh, &vl);
+        const float x = row_ok ? (i < 4 ? x0[i & 3] : x1[i & 3]) : 0.0f;
+        split2(GG ? x * q_sc : x, &vh, &vl);
         qh[rt][ks][i] = vh;
         ql[rt][ks][i] = vl;
       }
@@ -272,6 +296,8 @@ __global__ void __launch_bounds__(kPW * 64, 1)
   }
   float4_t sacc[RT][4];
   half8_t ph[RT][2], pl[RT][2];
+  u32x2 mk[RT][4];                             // GG: the lane's mask values of the tile
+  int vexp = -40;                              // GG: weights times radii carry 2^-vexp
 
   // Copies of 1 KB segments: wave w of NW takes every NW-th (a compile-time
   // count). The radii come with the keys, as Y(it) reads them before V(it)
@@ -290,6 +316,18 @@ __global__ void __launch_bounds__(kPW * 64, 1)
     constexpr int NW = decltype(nwc)::value;
 #pragma unroll
     for (int j = 0; j < P::VSEG / NW; ++j) copy_seg(vt[it & 1], it * P::BYTES + P::KBYTES, w + NW * j);
+  };
+
+  // GG: four tokens' values of each row and 16-token group (S is a multiple of
+  // four; the groups past it read the last four and are masked by their position)
+  auto load_mask = [&](int it) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt) {
+        const int t = min(it * kPT + 16 * tt + 4 * grp, a.S - 4);
+        mk[rt][tt] = a.mask != nullptr ? *(const u32x2 *)(mrow[rt] + t) : (u32x2){0u, 0u};
+      }
   };
 
   // The operands of a product step are read AHEAD steps before it (the fence
@@ -317,9 +355,10 @@ __global__ void __launch_bounds__(kPW * 64, 1)
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
-        sacc[rt][tt] = mfma16(ah[c], qh[rt][ks], sacc[rt][tt]);
+        if (!GG) sacc[rt][tt] = mfma16(ah[c], qh[rt][ks], sacc[rt][tt]);
         sacc[rt][tt] = mfma16(al[c], qh[rt][ks], sacc[rt][tt]);
         sacc[rt][tt] = mfma16(ah[c], ql[rt][ks], sacc[rt][tt]);
+        if (GG) sacc[rt][tt] = mfma16(ah[c], qh[rt][ks], sacc[rt][tt]);   // the small products first
       }
     }
   };
@@ -327,6 +366,7 @@ __global__ void __launch_bounds__(kPW * 64, 1)
     const uint8_t *t = vt[it & 1] + 16 * lane;
     auto op = [&](int n, int plane) { return *(lds_chalf8 *)(t + P::vseg(n >> 1, n & 1, plane) * 1024); };
     half8_t bh[AHEAD + 1], bl[AHEAD + 1];
+    float4_t part[RT];
 #pragma unroll
     for (int n = 0; n < AHEAD; ++n) {
       bh[n] = op(n, 0);
@@ -342,15 +382,35 @@ __global__ void __launch_bounds__(kPW * 64, 1)
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
-        oacc[rt][nb] = mfma16(ph[rt][kk], bh[c], oacc[rt][nb]);
-        oacc[rt][nb] = mfma16(ph[rt][kk], bl[c], oacc[rt][nb]);
-        oacc[rt][nb] = mfma16(pl[rt][kk], bh[c], oacc[rt][nb]);
+        // GG, whose results stay fp32: the tile's sum first, so that the long
+        // accumulation rounds once per tile instead of six times
+        float4_t &o = GG ? part[rt] : oacc[rt][nb];
+        if (GG && kk == 0) o = (float4_t){0.f, 0.f, 0.f, 0.f};
+        if (!GG) o = mfma16(ph[rt][kk], bh[c], o);
+        o = mfma16(ph[rt][kk], bl[c], o);
+        o = mfma16(pl[rt][kk], bh[c], o);
+        if (GG) o = mfma16(ph[rt][kk], bh[c], o);
+        if (GG && kk == 1) oacc[rt][nb] += o;
       }
     }
   };
   auto softmax = [&](int it) {
     const int t0 = it * kPT;
     const float *rk = rads[it % 3] + 4 * grp, *rv = rk + kPT;
+    float shrink = 1.0f, v_sc = 1.0f;
+    if constexpr (GG) {
+      float rmax = 0.0f;
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) rmax = fmaxf(rmax, rv[16 * tt + i]);
+      // the tile's largest radius below 2^14 (the same in every lane)
+      const int ex = (int)(__builtin_bit_cast(uint32_t, rows_max(rmax)) >> 23) & 0xFF;
+      const int need = max(vexp, __builtin_amdgcn_readfirstlane(ex) - 127 - 13);
+      shrink = __builtin_ldexpf(1.0f, vexp - need);
+      vexp = need;
+      v_sc = __builtin_ldexpf(1.0f, -vexp);
+    }
     const bool need_mask = t0 + kPT > a.S || (a.causal && t0 + kPT - 1 > a.q_start + q0);
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
@@ -359,7 +419,12 @@ __global__ void __launch_bounds__(kPW * 64, 1)
       for (int tt = 0; tt < 4; ++tt) {
         const float4_t r4 = *(const float4_t *)(rk + 16 * tt);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s[tt][i] = sacc[rt][tt][i] * r4[i];
+        for (int i = 0; i < 4; ++i) {
+          s[tt][i] = sacc[rt][tt][i] * r4[i];
+          if constexpr (GG)   // the mask in the exp2 domain
+            s[tt][i] = __builtin_fmaf(half_bits_to_float((uint16_t)(mk[rt][tt][i >> 1] >> (16 * (i & 1)))),
+                                      1.4426950408889634f, s[tt][i] * q_un[rt]);
+        }
       }
       if (need_mask) {
         const int last = a.causal ? min(a.S - 1, row_pos[rt]) : a.S - 1;   // last token this row sees
@@ -389,15 +454,16 @@ __global__ void __launch_bounds__(kPW * 64, 1)
           const float p = __builtin_amdgcn_exp2f(s[tt][i] - ref);
           psum += p;
           half_t vh, vl;
-          split2(p * r4[i], &vh, &vl);
+          split2(GG ? p * (r4[i] * v_sc) : p * r4[i], &vh, &vl);
           ph[rt][tt >> 1][4 * (tt & 1) + i] = vh;
           pl[rt][tt >> 1][4 * (tt & 1) + i] = vl;
         }
       }
       l_run[rt] = l_run[rt] * alpha + psum;
-      if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+      const float fade = GG ? alpha * shrink : alpha;
+      if (__builtin_amdgcn_ballot_w64(fade != 1.0f) != 0) {
         float f[4];
-        per_row(alpha, grp, f);
+        per_row(fade, grp, f);
 #pragma unroll
         for (int nb = 0; nb < NT; ++nb)
 #pragma unroll
@@ -415,6 +481,7 @@ __global__ void __launch_bounds__(kPW * 64, 1)
     // X(it1), values alone, stands after the loop: with it inside, behind a
     // condition, the scores would count as live across iterations
     auto x_stage = [&](int it) {
+      if constexpr (GG) load_mask(it);          // there by softmax(it)
       __builtin_amdgcn_s_setprio(1);
       if (it > it0) values(it - 1);
       __builtin_amdgcn_sched_barrier(0);
@@ -460,14 +527,18 @@ __global__ void __launch_bounds__(kPW * 64, 1)
     if (splits > 1 && grp == 0)
       ((float2 *)a.part_ml)[(prow0 + 32 * wave + 16 * rt + col) * splits + sp] = make_float2(m_run[rt], l);
     float f[4];
-    per_row(splits > 1 ? 1.0f : l > 0.0f ? 1.0f / (l * kPlaneScale) : 0.0f, grp, f);   // the value planes' 2^6 as well
+    float norm = splits > 1 ? 1.0f : l > 0.0f ? 1.0f / (l * kPlaneScale) : 0.0f;       // the value planes' 2^6 as well
+    if constexpr (GG) norm = __builtin_ldexpf(norm, vexp);
+    per_row(norm, grp, f);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int row = 32 * wave + 16 * rt + 4 * grp + i;
       const int tok = q0 + row / G;
       float *dst;
       if (splits > 1) dst = a.part_o + ((prow0 + row) * splits + sp) * D + col;
-      else if (row < a.qt * G && tok < a.Sq) dst = a.o + ((int64_t)(b * a.Hq + h * G + row % G) * a.Sq + tok) * D + col;
+      else if (row < a.qt * G && tok < a.Sq)
+        dst = a.o + (GG ? ((int64_t)b * a.Sq + tok) * a.Hq + h * G + row % G
+                        : (int64_t)(b * a.Hq + h * G + row % G) * a.Sq + tok) * D + col;
       else continue;
 #pragma unroll
       for (int nb = 0; nb < NT; ++nb) dst[16 * nb] = oacc[rt][nb][i] * f[i];
@@ -486,7 +557,9 @@ static hipError_t launch_planes_d(const PrefillArgs &a, int kb, int vb, const Pr
   else plane_decode_kernel<D, 2, 2><<<dg, 256, 0, s>>>(a, records, p.stream_bytes, stream0);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  prefill_planes_kernel<D><<<a.qtiles * a.splits * ns, kPW * 64, 0, s>>>(a, records, p.stream_bytes, stream0, ns);
+  const int blocks = a.qtiles * a.splits * ns;
+  if (a.token_major) prefill_planes_kernel<D, true><<<blocks, kPW * 64, 0, s>>>(a, records, p.stream_bytes, stream0, ns);
+  else prefill_planes_kernel<D, false><<<blocks, kPW * 64, 0, s>>>(a, records, p.stream_bytes, stream0, ns);
   e = hipGetLastError();
   if (e != hipSuccess || a.splits == 1) return e;
   return launch_prefill_merge(a, stream0, ns, kPRows, s);
