@@ -754,11 +754,12 @@ PrefillPlan prefill_plan(int B, int Hq, int Hkv, int Sq, int S, int d, bool qjl,
   const int G = Hq / Hkv;
   p.rows = prefill_rows_per_block(qjl);
   p.qt = p.rows / G;
-  p.qtiles = (Sq + p.qt - 1) / p.qt;
+  p.qtiles = (Sq - 1) / p.qt + 1;
   p.splits = 1;
-  p.streams = B * Hkv;
+  const int64_t all = (int64_t)B * Hkv;
+  p.streams = (int)(all < 0x7fffffff ? all : 0x7fffffff);
   if (!extra || S < 1) return p;
-  const int tiles = (S + kPT - 1) / kPT;
+  const int tiles = (S - 1) / kPT + 1;   // (a size query may ask for any int)
   // Decoding each tile once per call instead of once per row block pays from
   // some row blocks on (records are written and read back, 1 KB per token at
   // d = 128). Whole calls, decoded once / per row block: d = 128 12 row blocks
@@ -770,7 +771,7 @@ PrefillPlan prefill_plan(int B, int Hq, int Hkv, int Sq, int S, int d, bool qjl,
   p.planes = !qjl && (planes_only || p.qtiles >= (d == 128 ? 12 : 6)) && p.stream_bytes <= kPlaneBudget;
   if (p.planes) {
     // equal passes over the streams
-    const int64_t all = p.streams, fit = kPlaneBudget / p.stream_bytes, passes = (all + fit - 1) / fit;
+    const int64_t fit = kPlaneBudget / p.stream_bytes, passes = (all + fit - 1) / fit;
     p.streams = (int)((all + passes - 1) / passes);
   }
   const int64_t blocks = (int64_t)p.qtiles * p.streams;

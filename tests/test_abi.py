@@ -144,6 +144,23 @@ def test_prefill_validation():
     assert _prefill(Sq=0) == 0                                 # nothing to do
 
 
+def test_prefill_workspace_queries_take_any_shape():
+    """Counts whose products or round-ups leave 32 bits give a size, not an
+    abort: streams, query tokens, cached tokens, and a stream whose decoded
+    tiles exceed their budget, which keeps the kernel that decodes per row block."""
+    L = _lib.lib()
+    top = 2 ** 31 - 1
+    for shape in ((65536, 65536, 65536, 1, 64, 128), (1 << 15, 1 << 16, 1 << 16, 800, 64, 64), (1, 4, 1, 4096, top, 128),
+                  (1, 1, 1, top, 64, 128), (top, top, top, 1, top, 64), (1, 4, 1, 800, 2081100, 128)):
+        base = L.pqkv_prefill_workspace_bytes(*shape)
+        for qjl in (0, 1):
+            extra = L.pqkv_prefill_workspace_preferred_bytes(*shape, qjl) - base
+            assert 0 <= extra <= (2 << 30) + (40 << 20), (shape, qjl, extra)
+    # 32 513 tiles of 66 048 bytes fit 2 GiB, one more does not
+    fits, not_ = (L.pqkv_prefill_workspace_preferred_bytes(1, 4, 1, 800, n, 128, 0) for n in (32513 * 64, 32513 * 64 + 1))
+    assert fits > 2 << 30 > not_
+
+
 def test_zero_sized_calls_are_no_ops():
     L = _lib.lib()
     assert L.pqkv_rotate(None, 0, None, None, 0, 0, 128, 0, None) == 0
