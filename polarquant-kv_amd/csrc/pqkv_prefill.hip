@@ -49,17 +49,14 @@
 // final normalisation (/ 2^6).
 #include "pqkv_device.h"
 #include "pqkv_launch.h"
+#include "pqkv_prefill.h"
 
 namespace pqkv {
 
 namespace {
 
-constexpr int kPW = 8;                    // waves per workgroup
 constexpr int kPRowsWave = 32;            // query rows per wave
-constexpr int kPT = 64;                   // kv tokens per tile
 constexpr int kSegBytes = 64 * 8;         // one operand segment: 64 lanes x 8 bytes
-constexpr float kPlaneScale = kPrefillPlaneScale;              // codebook planes and queries, x 2^6
-constexpr float kScoreUnscale = 1.0f / (kPlaneScale * kPlaneScale);
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
@@ -67,16 +64,6 @@ typedef __attribute__((address_space(3))) const u32x2 lds_cu32x2;
 
 __device__ __forceinline__ void lds_put8(uint8_t *p, uint32_t a, uint32_t b) { *(lds_u32x2 *)p = (u32x2){a, b}; }
 __device__ __forceinline__ u32x2 lds_get8(const uint8_t *p) { return *(lds_cu32x2 *)p; }
-
-// x is made opaque first: otherwise the compiler rounds a product once for lo's
-// hi (v_fma_mixlo_f16) and twice for the stored one, and where they differ the
-// pair is off by an fp16 step (1e-3 of a weight, in one of some thousands).
-__device__ __forceinline__ void split2(float x, half_t *hi, half_t *lo) {
-  asm("" : "+v"(x));
-  const half_t h = (half_t)x;
-  *hi = h;
-  *lo = (half_t)(x - (float)h);
-}
 
 __device__ __forceinline__ uint32_t pack_h2(half_t a, half_t b) {
   half2_t v = {a, b};
@@ -87,31 +74,6 @@ __device__ __forceinline__ half8_t pack8u(u32x2 a, u32x2 b) {
   typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
   u32x4v v = {a.x, a.y, b.x, b.y};
   return __builtin_bit_cast(half8_t, v);
-}
-
-__device__ __forceinline__ float4_t mfma16(half8_t a, half8_t b, float4_t c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-
-__device__ __forceinline__ float rows_max(float x) {
-  auto a = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
-  x = fmaxf(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
-  auto b = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
-  return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
-}
-__device__ __forceinline__ float rows_sum(float x) {
-  auto a = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
-  x = __builtin_bit_cast(float, (uint32_t)a[0]) + __builtin_bit_cast(float, (uint32_t)a[1]);
-  auto b = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
-  return __builtin_bit_cast(float, (uint32_t)b[0]) + __builtin_bit_cast(float, (uint32_t)b[1]);
-}
-
-// Value of lane `row` (0..15) for output row 4 grp + i (v is the same in
-// the four lanes of a column): one lane gather per i.
-__device__ __forceinline__ void per_row(float v, int grp, float (&f)[4]) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    f[i] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * (4 * grp + i), __builtin_bit_cast(int, v)));
 }
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t stream_rsrc(const uint8_t *base, uint32_t bytes) {

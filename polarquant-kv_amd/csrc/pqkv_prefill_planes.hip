@@ -45,16 +45,13 @@
 
 #include "pqkv_device.h"
 #include "pqkv_launch.h"
+#include "pqkv_prefill.h"
 
 namespace pqkv {
 
 namespace {
 
-constexpr int kPT = 64;                        // kv tokens per tile
-constexpr int kPW = 8;                         // waves per workgroup
 constexpr int kPRows = 32 * kPW;               // query rows per workgroup
-constexpr float kPlaneScale = kPrefillPlaneScale;
-constexpr float kScoreUnscale = 1.0f / (kPlaneScale * kPlaneScale);
 
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(3))) const half8_t lds_chalf8;
@@ -72,41 +69,6 @@ struct PlaneRec {
   __host__ __device__ static constexpr int kseg(int tt, int ks, int plane) { return (tt * KS + ks) * 2 + plane; }
   __host__ __device__ static constexpr int vseg(int nb, int kk, int plane) { return (nb * 2 + kk) * 2 + plane; }
 };
-
-// x is made opaque first: otherwise the compiler rounds a product once for lo's
-// hi (v_fma_mixlo_f16) and twice for the stored one, and where they differ the
-// pair is off by an fp16 step (1e-3 of a weight, in one of some thousands).
-__device__ __forceinline__ void split2(float x, half_t *hi, half_t *lo) {
-  asm("" : "+v"(x));
-  const half_t h = (half_t)x;
-  *hi = h;
-  *lo = (half_t)(x - (float)h);
-}
-
-__device__ __forceinline__ float4_t mfma16(half8_t a, half8_t b, float4_t c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-
-// max / sum of a value over the four lanes of a column (l, l ^ 16, l ^ 32, l ^ 48)
-__device__ __forceinline__ float rows_max(float x) {
-  auto a = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
-  x = fmaxf(__builtin_bit_cast(float, (uint32_t)a[0]), __builtin_bit_cast(float, (uint32_t)a[1]));
-  auto b = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
-  return fmaxf(__builtin_bit_cast(float, (uint32_t)b[0]), __builtin_bit_cast(float, (uint32_t)b[1]));
-}
-__device__ __forceinline__ float rows_sum(float x) {
-  auto a = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
-  x = __builtin_bit_cast(float, (uint32_t)a[0]) + __builtin_bit_cast(float, (uint32_t)a[1]);
-  auto b = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
-  return __builtin_bit_cast(float, (uint32_t)b[0]) + __builtin_bit_cast(float, (uint32_t)b[1]);
-}
-// Value of lane `row` (0..15) for output row 4 grp + i (v is the same in the
-// four lanes of a column): one lane gather per i.
-__device__ __forceinline__ void per_row(float v, int grp, float (&f)[4]) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    f[i] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * (4 * grp + i), __builtin_bit_cast(int, v)));
-}
 
 __device__ __forceinline__ uint32_t load_u32_any(const uint8_t *p) {   // 2-byte aligned
   return (uint32_t)((const uint16_t *)p)[0] | ((uint32_t)((const uint16_t *)p)[1] << 16);
