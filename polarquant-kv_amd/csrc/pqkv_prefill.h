@@ -24,6 +24,19 @@ __device__ __forceinline__ void split2(float x, half_t *hi, half_t *lo) {
   *lo = (half_t)(x - (float)h);
 }
 
+// The same of two products a b, as packed pairs: lo is taken from the exact
+// product (a mixed fused multiply-add), so a pair also holds what rounding the
+// product lost. The hi halves are made opaque, which keeps one rounding of each.
+// With the products opaque instead, which costs a widening and a subtraction per
+// weight, a prefill of 509 tokens against 32 000 cached ones (batch 32, 32 query
+// / 8 kv heads, d = 128) takes 22.6 ms in place of 21.5.
+__device__ __forceinline__ void split2_products(float a0, float b0, float a1, float b1, half2_t *hi, half2_t *lo) {
+  half2_t h = {(half_t)(a0 * b0), (half_t)(a1 * b1)};
+  asm("" : "+v"(h));
+  *hi = h;
+  *lo = half2_t{(half_t)__builtin_fmaf(a0, b0, -(float)h[0]), (half_t)__builtin_fmaf(a1, b1, -(float)h[1])};
+}
+
 __device__ __forceinline__ float4_t mfma16(half8_t a, half8_t b, float4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }

@@ -508,15 +508,19 @@ __global__ void __launch_bounds__(kPW * 64, 1) prefill_mfma_kernel(const Prefill
         const float4 r4 = *(const float4 *)&rv[16 * tt + 4 * grp];
         const float rr[4] = {r4.x, r4.y, r4.z, r4.w};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float p = __builtin_amdgcn_exp2f(s[tt][i] - ref);
-          psum += p;
-          half_t vh, vl;
-          split2(p * rr[i], &vh, &vl);
+        for (int i = 0; i < 4; i += 2) {
+          const float p0 = __builtin_amdgcn_exp2f(s[tt][i] - ref), p1 = __builtin_amdgcn_exp2f(s[tt][i + 1] - ref);
+          psum += p0;
+          psum += p1;
+          half2_t vh, vl;
+          split2_products(p0, rr[i], p1, rr[i + 1], &vh, &vl);
           // A operand of the value product: k = 8 grp + i' <-> token tile
           // 2 kk + i' / 4, token 4 grp + i' % 4
-          ph[rt][tt >> 1][4 * (tt & 1) + i] = vh;
-          pl[rt][tt >> 1][4 * (tt & 1) + i] = vl;
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            ph[rt][tt >> 1][4 * (tt & 1) + i + e] = vh[e];
+            pl[rt][tt >> 1][4 * (tt & 1) + i + e] = vl[e];
+          }
         }
       }
       l_run[rt] = l_run[rt] * alpha + psum;
