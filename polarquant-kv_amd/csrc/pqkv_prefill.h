@@ -14,6 +14,9 @@ constexpr int kPW = 8;                    // waves per workgroup
 constexpr float kPlaneScale = kPrefillPlaneScale;              // codebook planes and queries, x 2^6
 constexpr float kScoreUnscale = 1.0f / (kPlaneScale * kPlaneScale);
 
+// four floats on a dword boundary
+typedef float float4_dw __attribute__((ext_vector_type(4), aligned(4)));
+
 // x is made opaque first: otherwise the compiler rounds a product once for lo's
 // hi (v_fma_mixlo_f16) and twice for the stored one, and where they differ the
 // pair is off by an fp16 step (1e-3 of a weight, in one of some thousands).
@@ -39,6 +42,13 @@ __device__ __forceinline__ void split2_products(float a0, float b0, float a1, fl
 
 __device__ __forceinline__ float4_t mfma16(half8_t a, half8_t b, float4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+
+// First tile of share sp when `all` tiles are cut into `splits` shares:
+// floor(all sp / splits), without the 64-bit division.
+__host__ __device__ __forceinline__ int share_begin(int all, int sp, int splits) {
+  const int q = all / splits, r = all - q * splits;
+  return q * sp + r * sp / splits;
 }
 
 // max / sum of a value over the four lanes of a column (l, l ^ 16, l ^ 32, l ^ 48)

@@ -203,7 +203,7 @@ __global__ void __launch_bounds__(kPW * 64, 1)
   const int q_last = min(a.Sq, q0 + a.qt) - 1;
   const int kv_end = a.causal ? min(a.S, a.q_start + q_last + 1) : a.S;
   const int all = (kv_end + kPT - 1) / kPT;
-  const int it0 = (int)((int64_t)all * sp / splits), it1 = (int)((int64_t)all * (sp + 1) / splits);
+  const int it0 = share_begin(all, sp, splits), it1 = share_begin(all, sp + 1, splits);
 
   const uint8_t *stream = planes + (int64_t)sl * stream_bytes;
   const __amdgpu_buffer_rsrc_t res =
