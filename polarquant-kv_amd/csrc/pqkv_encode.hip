@@ -195,7 +195,27 @@ struct RowsSource {
     return x[sq * s_s + h * s_h + iq * s_q + j];
   }
 };
-template <int D, bool INVERSE, typename SRC, typename TOUT>
+// Block-encoded vectors (block_pq4 / block_pq2), rows of n_inner of them
+// outer_stride bytes apart: r16 c[code], the rotated reconstruction the
+// attention kernels use.
+template <int D, int BITS>
+struct BlockSource {
+  const uint8_t *blocks;
+  const float *cb;
+  int64_t outer_stride;
+  FastDiv by_inner;
+  __device__ __forceinline__ float operator()(int64_t v, int j) const {
+    const uint32_t o = by_inner.div((uint32_t)v), vi = (uint32_t)v - o * by_inner.d;
+    const uint8_t *vec = blocks + o * outer_stride + (int64_t)vi * vector_bytes(D, BITS);
+    const float r = half_bits_to_float(*(const uint16_t *)vec);
+    constexpr int per = 8 / BITS;                          // codes per byte
+    const uint8_t byte = vec[qs_offset(j / per, BITS)];
+    return r * cb[(byte >> (BITS * (j % per))) & ((1 << BITS) - 1)];
+  }
+};
+// SAT16: fp16 output saturates at +-65504 like the reference's decompress
+// (decompress_kernel.py:52-55, clamp(-65504, 65504).half()).
+template <int D, bool INVERSE, typename SRC, typename TOUT, bool SAT16 = false>
 __global__ void __launch_bounds__(256) rotate_kernel(const SRC src, const float *__restrict__ R,
                                                      TOUT *__restrict__ y, int64_t n, float out_scale) {
   constexpr int RP = D + 4;
@@ -254,7 +274,9 @@ __global__ void __launch_bounds__(256) rotate_kernel(const SRC src, const float 
     }
     const int64_t v = base + g;
     if (v < n) {
-      y[v * D + c0 + jj] = (TOUT)(acc * out_scale);
+      float o = acc * out_scale;
+      if (SAT16) o = o > 65504.0f ? 65504.0f : (o < -65504.0f ? -65504.0f : o);
+      y[v * D + c0 + jj] = (TOUT)o;
     }
     __syncthreads();
   }
@@ -652,6 +674,28 @@ hipError_t launch_rotate_rows(const float *x, int64_t s_q, int64_t s_h, int64_t 
     const dim3 grid(grid_for(n, kRotVec, 2048), 64 / kRotCols);
     rotate_kernel<64, false, RowsSource, float><<<grid, 256, 0, s>>>(src, R, y, n, out_scale);
   }
+  return hipGetLastError();
+}
+
+template <int D, int BITS>
+static void dequant_dispatch(const uint8_t *blocks, int64_t stride, const float *cb, const float *R, void *y, int yt,
+                             int64_t n_outer, int64_t n_inner, hipStream_t s) {
+  const int64_t n = n_outer * n_inner;
+  const dim3 grid(grid_for(n, kRotVec, 2048), D / kRotCols);
+  using S = BlockSource<D, BITS>;
+  const S src{blocks, cb, stride, FastDiv((uint32_t)n_inner)};
+  if (yt == 0) rotate_kernel<D, true, S, float><<<grid, 256, 0, s>>>(src, R, (float *)y, n, 1.0f);
+  else rotate_kernel<D, true, S, half_t, true><<<grid, 256, 0, s>>>(src, R, (half_t *)y, n, 1.0f);
+}
+
+hipError_t launch_dequantize_few(const uint8_t *blocks, int64_t blocks_outer_stride, const float *codebook, int bits,
+                                 const float *R, void *y, int y_dtype, int64_t n_outer, int64_t n_inner, int d,
+                                 hipStream_t s) {
+  const int64_t st = blocks_outer_stride;
+  if (d == 128 && bits == 4) dequant_dispatch<128, 4>(blocks, st, codebook, R, y, y_dtype, n_outer, n_inner, s);
+  else if (d == 128) dequant_dispatch<128, 2>(blocks, st, codebook, R, y, y_dtype, n_outer, n_inner, s);
+  else if (bits == 4) dequant_dispatch<64, 4>(blocks, st, codebook, R, y, y_dtype, n_outer, n_inner, s);
+  else dequant_dispatch<64, 2>(blocks, st, codebook, R, y, y_dtype, n_outer, n_inner, s);
   return hipGetLastError();
 }
 

@@ -219,6 +219,11 @@ hipError_t launch_rotate_rows_mfma(const float *x, int64_t s_q, int64_t s_h, int
 hipError_t launch_dequantize(const uint8_t *blocks, int64_t blocks_outer_stride, const float *codebook, int bits,
                              const float *R, void *y, int y_dtype, int64_t y_outer_stride, int64_t n_outer,
                              int64_t n_inner, int d, hipStream_t s);
+// The same without the matrix cores, for few vectors (n_outer n_inner below
+// 2^32) into one run of outputs: the same bits.
+hipError_t launch_dequantize_few(const uint8_t *blocks, int64_t blocks_outer_stride, const float *codebook, int bits,
+                                 const float *R, void *y, int y_dtype, int64_t n_outer, int64_t n_inner, int d,
+                                 hipStream_t s);
 hipError_t launch_encode_exact(const EncodeArgs &a, int x_dtype, hipStream_t s);
 // The exact encoder on the fp32 matrix cores (same rotation, same indices) for
 // inputs it reads in 16-byte pieces; the exact launchers take it where

@@ -270,7 +270,14 @@ hipError_t launch_dequantize(const uint8_t *blocks, int64_t blocks_outer_stride,
     const uint8_t *b = blocks + o * blocks_outer_stride;
     void *yo = (uint8_t *)y + o * y_outer_stride * ys;
     hipError_t e;
-    if (d == 128 && bits == 4) e = dequant_d<128, 4>(b, blocks_outer_stride, codebook, R, yo, y_dtype, no, n_inner, s);
+    // Few vectors spread over more compute units in the kernel of 8 vectors by
+    // 32 columns (32 or 64 vectors by all columns here). Measured crossover
+    // (4-bit, fp16 out, replayed graphs, there / here): d = 128 3.0 / 4.7 us
+    // for 1 vector, 4.2 / 5.0 for 1024, 5.6 / 4.8 for 1792; d = 64 2.5 / 3.6
+    // for 1, 3.0 / 3.7 for 2048, 3.6 / 3.7 for 4096, 3.95 / 3.7 for 4608.
+    if (no * n_inner <= (d == 128 ? 1024 : 4096))
+      e = launch_dequantize_few(b, blocks_outer_stride, codebook, bits, R, yo, y_dtype, no, n_inner, d, s);
+    else if (d == 128 && bits == 4) e = dequant_d<128, 4>(b, blocks_outer_stride, codebook, R, yo, y_dtype, no, n_inner, s);
     else if (d == 128) e = dequant_d<128, 2>(b, blocks_outer_stride, codebook, R, yo, y_dtype, no, n_inner, s);
     else if (bits == 4) e = dequant_d<64, 4>(b, blocks_outer_stride, codebook, R, yo, y_dtype, no, n_inner, s);
     else e = dequant_d<64, 2>(b, blocks_outer_stride, codebook, R, yo, y_dtype, no, n_inner, s);

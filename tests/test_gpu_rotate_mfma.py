@@ -94,3 +94,38 @@ def test_dequantize_rows_bits(d, bits, B, H, S, cap):
     mixed.blocks.copy_(wide[:, :H].reshape(B, -1))
     mixed.seq_len = S
     assert torch.equal(_bits(quantizer.dequantize(mixed, Rt, torch.float32)), _bits(got))
+
+
+def _block_cache(B, H, S, cap, d, bits):
+    """A cache whose first S positions hold random codes and radii, and the
+    same vectors one after the other."""
+    g = torch.Generator().manual_seed(d + bits + S)
+    cache = quantizer.allocate_cache(B, H, cap, d, bits, DEV)
+    cache.blocks.copy_(torch.randint(0, 256, cache.blocks.shape, generator=g, dtype=torch.uint8))
+    r = (torch.randn(B, H, cap, 1, 1, generator=g) * 2).exp().half().view(torch.uint8).to(DEV)
+    cache.blocks.unflatten(-1, (d // 32, -1))[..., :2] = r.reshape(B, H, cap, 1, 2)
+    cache.seq_len = S
+    return cache, cache.blocks[:, :, :S].reshape(B * H * S, -1)
+
+
+def _in_chunks(rows, R, codebook, bits, d, dtype, step):
+    out = torch.empty(rows.shape[0], d, dtype=dtype, device=DEV)
+    for i in range(0, rows.shape[0], step):
+        n = min(step, rows.shape[0] - i)
+        _lib.check(_lib.lib().pqkv_dequantize(rows[i:].data_ptr(), codebook.data_ptr(), bits, R.data_ptr(),
+                                              out[i:].data_ptr(), _lib.dtype_code(dtype), n, d, _lib.stream_of(out)))
+    return out
+
+
+@pytest.mark.parametrize("d,bits", [(64, 2), (64, 4), (128, 2), (128, 4)])
+@pytest.mark.parametrize("B,H,S,cap", [(1, 1, 1024, 1024), (5, 1, 205, 300), (2, 2, 256, 257), (1, 8, 512, 520),
+                                       (1, 17, 241, 250)])
+def test_dequantize_bits_on_both_sides_of_the_line(d, bits, B, H, S, cap):
+    """1024 / 1025 vectors at d = 128, 4096 / 4097 at d = 64, rows apart: every
+    bit is what one vector at a time gives (few vectors: the vector ALU kernel)."""
+    print(f"dequantize line d={d} bits={bits} B={B} H={H} S={S}", flush=True)
+    cache, rows = _block_cache(B, H, S, cap, d, bits)
+    R = torch.from_numpy(O.rotation_matrix(d, 42).astype(np.float32)).to(DEV)
+    for dtype in (torch.float16, torch.float32):
+        got = quantizer.dequantize(cache, R, dtype).reshape(-1, d)
+        assert torch.equal(_bits(got), _bits(_in_chunks(rows, R, cache.codebooks, bits, d, dtype, 333)))
