@@ -359,12 +359,14 @@ __global__ void __launch_bounds__(256) rotate2_kernel(const TIN *__restrict__ x,
 
 // Many vectors (on a 16-byte boundary) go to the fp32 matrix cores, the same
 // bits. Measured crossover (fp16 -> fp32, replayed graphs): d = 128 3.7 us here
-// against 4.7 us there at 1024 vectors, 5.0 against 4.8 at 2048, 12.1 against
-// 5.3 at 8192, 392 against 103 at 400 000; d = 64 2.7 against 3.1 at 2048, 3.6
-// against 3.2 at 4096, 107 against 32 at 400 000. Below it the launch spreads
-// over too few compute units there (32 or 64 vectors per workgroup, 8 here).
+// against 4.7 us there at 1024 vectors, 4.9 against 4.9 at 2048 (one round of
+// workgroups here; fp32 input 4.4 against 4.9, and 4.9 against 4.9 at 2176),
+// 12.1 against 5.3 at 8192, 392 against 103 at 400 000; d = 64 2.7 against 3.1
+// at 2048, 3.3 against 3.3 at 4096, 107 against 32 at 400 000. Below it the
+// launch spreads over too few compute units there (32 or 64 vectors per
+// workgroup, 8 here).
 static bool rotate_mfma_ok(const void *x, int64_t n, int d) {
-  return n >= (d == 128 ? 2048 : 4096) && (uintptr_t)x % 16 == 0;
+  return n > (d == 128 ? 2048 : 4096) && (uintptr_t)x % 16 == 0;
 }
 
 hipError_t launch_rotate2(const void *x, int x_dtype, const float *R, const float *M, float *y, float *z, int64_t n,
