@@ -936,10 +936,10 @@ int prefill_attn_run(const void *q, int q_dtype, const float *R, const uint8_t *
   const size_t need = pqkv_prefill_workspace_bytes(B, Hq, Hkv, Sq, S, d);
   if (!workspace || workspace_bytes < need)
     return fail(PQKV_ERR_WORKSPACE, "prefill: workspace %zu < %zu bytes", workspace_bytes, need);
-  // the faster plan if the workspace holds what it needs, else one workgroup
-  // per row block that decodes the tiles itself
+  // the faster plan if the workspace holds what it needs (on a 16-byte
+  // boundary), else one workgroup per row block that decodes the tiles itself
   pqkv::PrefillPlan plan = pqkv::prefill_plan(B, Hq, Hkv, Sq, S, d, qjl, true);
-  if (workspace_bytes < need + plan.bytes(d)) plan = pqkv::prefill_plan(B, Hq, Hkv, Sq, S, d, qjl, false);
+  if ((uintptr_t)workspace % 16 || workspace_bytes < need + plan.bytes(d)) plan = pqkv::prefill_plan(B, Hq, Hkv, Sq, S, d, qjl, false);
   float *part = (float *)((char *)workspace + need);
   uint8_t *records = (uint8_t *)part + plan.part_bytes(d);
   float *q32 = (float *)workspace;

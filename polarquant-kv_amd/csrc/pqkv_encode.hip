@@ -371,7 +371,7 @@ static bool rotate_mfma_ok(const void *x, int64_t n, int d) {
 
 hipError_t launch_rotate2(const void *x, int x_dtype, const float *R, const float *M, float *y, float *z, int64_t n,
                           int d, float sy, float sz, hipStream_t s) {
-  if (rotate_mfma_ok(x, n, d)) {
+  if (rotate_mfma_ok(x, n, d) && (uintptr_t)y % 16 == 0) {   // (y is the second one's input)
     const hipError_t e = launch_rotate_mfma(x, x_dtype, R, y, 0, n, d, 0, sy, s);
     return e != hipSuccess ? e : launch_rotate_mfma(y, 0, M, z, 0, n, d, 0, sz, s);
   }

@@ -78,3 +78,51 @@ def test_split_equals_whole(B, Hq, Hkv, Sq, q_start, d, causal, kind):
     whole = _run(q, kc, vc, R, jl, q_start, causal, False)
     split = _run(q, kc, vc, R, jl, q_start, causal, True)
     _check(split, whole, vc if kind != "paged" else vc.to_contiguous(), R)
+
+
+def _call(q, kc, vc, R, jl, q_start, causal, ws):
+    """pqkv_prefill_attn on a workspace of the caller's (a uint8 tensor), fp32 out."""
+    B, Hq, Sq, d = q.shape
+    mixed = kc.mixed
+    kcb, vcb = attention._codebook_tables(kc, vc, mixed, kc.num_heads)
+    out = torch.empty(B, Hq, Sq, d, device=DEV)
+    _lib.check(_lib.lib().pqkv_prefill_attn(
+        q.data_ptr(), _lib.dtype_code(q.dtype), R.data_ptr(), kc.blocks.data_ptr(), vc.blocks.data_ptr(), kcb.data_ptr(),
+        vcb.data_ptr(), kc.head_bits()[0], vc.head_bits()[0], _lib.int_array(kc.head_bits()) if mixed else None,
+        _lib.int_array(vc.head_bits()) if mixed else None, _lib.ptr(kc.qjl_signs if jl is not None else None), _lib.ptr(jl),
+        d if jl is not None else 0, B, Hq, kc.num_heads, Sq, q_start, kc.seq_len, kc.max_seq_len, d, d ** -0.5, causal,
+        out.data_ptr(), _lib.F32, ws.data_ptr(), ws.numel(), _lib.stream_of(q)))
+    return out
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,q_start,d,qjl", [(1, 8, 2, 9, 1000, 128, False), (1, 8, 2, 801, 100, 128, False),
+                                                       (2, 32, 8, 40, 1000, 128, True), (2, 14, 2, 300, 1003, 64, False)])
+def test_workspace_off_a_16_byte_boundary(B, Hq, Hkv, Sq, q_start, d, qjl):
+    """A workspace on a dword boundary only, of any size, gives what the
+    smallest aligned one gives, bit for bit."""
+    print(f"prefill workspace + 4 bytes {B} {Hq} {Hkv} Sq={Sq} d={d} qjl={qjl}", flush=True)
+    S = q_start + Sq
+    R = torch.from_numpy(O.rotation_matrix(d, 42).astype(np.float32)).to(DEV)
+    jl = torch.from_numpy((O.jl_matrix(d, d, 43) @ O.rotation_matrix(d, 42).T).astype(np.float32)).to(DEV) if qjl else None
+    kc, vc = (quantizer.compress_pq(_states(B, Hkv, S, d, 5 + i), R, jl_rot=jl if i == 0 else None) for i in range(2))
+    q = torch.randn(B, Hq, Sq, d, generator=torch.Generator().manual_seed(S)).half().to(DEV)
+    L = _lib.lib()
+    base = L.pqkv_prefill_workspace_bytes(B, Hq, Hkv, Sq, S, d)
+    most = L.pqkv_prefill_workspace_preferred_bytes(B, Hq, Hkv, Sq, S, d, int(qjl))
+    assert most > base
+    want = _call(q, kc, vc, R, jl, q_start, 1, torch.empty(base, dtype=torch.uint8, device=DEV))
+    ws = torch.empty(most + 4, dtype=torch.uint8, device=DEV)
+    for n in (base, most):
+        assert torch.equal(_call(q, kc, vc, R, jl, q_start, 1, ws[4:4 + n]), want)
+
+
+def test_decode_workspace_off_a_16_byte_boundary():
+    """The same for the query rotations of a decode of many rows with sign corrections."""
+    B, Hq, Hkv, S, d = 66, 32, 8, 70, 128
+    R = torch.from_numpy(O.rotation_matrix(d, 42).astype(np.float32)).to(DEV)
+    jl = torch.from_numpy((O.jl_matrix(d, d, 43) @ O.rotation_matrix(d, 42).T).astype(np.float32)).to(DEV)
+    kc, vc = (quantizer.compress_pq(_states(B, Hkv, S, d, 5 + i), R, jl_rot=jl if i == 0 else None) for i in range(2))
+    q = torch.randn(B, Hq, d, generator=torch.Generator().manual_seed(S)).half().to(DEV)
+    ws = torch.empty(_lib.lib().pqkv_decode_workspace_bytes(B, Hq, Hkv, S, d) + 4, dtype=torch.uint8, device=DEV)
+    got = [attention.decode_attention(q, kc, vc, R, jl_rot=jl, out_dtype=torch.float32, workspace=w) for w in (ws[:-4], ws[4:])]
+    assert torch.equal(*got)
