@@ -215,27 +215,34 @@ def dequantize(cache: PQCache, rotation_matrix: torch.Tensor | None, out_dtype=t
     R = (torch.eye(d, device=dev) if rotation_matrix is None else rotation_matrix).to(torch.float32).contiguous()
     _lib.require_device(cache.blocks, R)
     out = torch.empty(B, H, S, d, dtype=out_dtype, device=dev)
-    if S == 0:
+    if out.numel() == 0:
         return out
+    if S > cache.max_seq_len:
+        raise ValueError(f"positions {S} exceed the cache capacity {cache.max_seq_len}")
     lib = _lib.lib()
     stream = _lib.stream_of(out)
     code = _lib.dtype_code(out_dtype)
+
+    def rows(blocks, stride, cb, bits, dst, dst_stride, n):
+        """n rows of S vectors `stride` bytes apart; a launch takes rows that
+        do not overlap, those of an expanded cache go one by one."""
+        one_launch = n == 1 or stride >= S * vector_bytes(d, bits)
+        for i in range(1 if one_launch else n):
+            _lib.check(lib.pqkv_dequantize_rows(blocks + i * stride, stride, cb.data_ptr(), bits, R.data_ptr(),
+                                                dst[i].data_ptr(), code, dst_stride, n if one_launch else 1, S, d, stream))
+
     if not cache.mixed:
         # every (batch, head) row of the cache, S_max vectors apart, in one
         # launch (one per batch row where the batch stride is its own)
         sb, sh = cache.blocks.stride(0), cache.blocks.stride(1)
-        rows, batches = (B * H, 1) if sb == H * sh else (H, B)
+        n, batches = (B * H, 1) if sb == H * sh else (H, B)
         for b in range(batches):
-            _lib.check(lib.pqkv_dequantize_rows(cache.blocks[b].data_ptr(), sh, cache.codebooks.data_ptr(),
-                                                cache.n_bits, R.data_ptr(), out[b].data_ptr(), code, S * d, rows, S, d,
-                                                stream))
+            rows(cache.blocks[b].data_ptr(), sh, cache.codebooks, cache.n_bits, out[b:].flatten(0, 1), S * d, n)
         return out
     for h, bits in enumerate(cache.head_bits()):
         # one head of every batch row per launch
         cb = cache.codebooks[h] if cache.codebooks.dim() == 2 else cache.codebooks
-        _lib.check(lib.pqkv_dequantize_rows(cache.blocks.data_ptr() + cache.head_offset(h), cache.blocks.stride(0),
-                                            cb.data_ptr(), bits, R.data_ptr(), out[:, h].data_ptr(), code, H * S * d,
-                                            B, S, d, stream))
+        rows(cache.blocks.data_ptr() + cache.head_offset(h), cache.blocks.stride(0), cb, bits, out[:, h], H * S * d, B)
     return out
 
 

@@ -129,3 +129,26 @@ def test_dequantize_bits_on_both_sides_of_the_line(d, bits, B, H, S, cap):
     for dtype in (torch.float16, torch.float32):
         got = quantizer.dequantize(cache, R, dtype).reshape(-1, d)
         assert torch.equal(_bits(got), _bits(_in_chunks(rows, R, cache.codebooks, bits, d, dtype, 333)))
+
+
+@pytest.mark.parametrize("bits", [4, (4, 2, 4)])
+def test_dequantize_of_empty_and_expanded_caches(bits):
+    """No batch rows give an empty result; a cache whose batch rows (or heads)
+    are one set of bytes expanded gives that set's values in each."""
+    d, S, cap = 128, 33, 40
+    R = torch.from_numpy(O.rotation_matrix(d, 42).astype(np.float32)).to(DEV)
+    one = quantizer.allocate_cache(1, 3, cap, d, bits, DEV)
+    x = torch.randn(1, 3, S, d, generator=torch.Generator().manual_seed(1)).to(DEV)
+    quantizer.compress_pq(x, R, cache=one, start=0)
+    want = quantizer.dequantize(one, R, torch.float32)
+    empty = quantizer.allocate_cache(0, 3, cap, d, bits, DEV)
+    assert quantizer.dequantize(empty, R, positions=S).shape == (0, 3, S, d)
+    beams = quantizer.allocate_cache(4, 3, cap, d, bits, DEV, codebooks=one.codebooks)
+    beams.blocks, beams.seq_len = one.blocks.expand(4, *one.blocks.shape[1:]), S
+    assert torch.equal(quantizer.dequantize(beams, R, torch.float32), want.expand(4, -1, -1, -1))
+    with pytest.raises(ValueError):
+        quantizer.dequantize(one, R, positions=cap + 1)
+    if bits == 4:
+        heads = quantizer.allocate_cache(2, 3, cap, d, bits, DEV)
+        heads.blocks, heads.seq_len = one.blocks[:, :1].expand(2, 3, -1, -1), S
+        assert torch.equal(quantizer.dequantize(heads, R, torch.float32), want[:, :1].expand(2, 3, -1, -1))
