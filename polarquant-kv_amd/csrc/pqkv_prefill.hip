@@ -714,38 +714,70 @@ constexpr int kTargetBlocks = 256;
 constexpr int64_t kPlaneBudget = (int64_t)2 << 30;   // bytes of decoded tiles at a time
 
 PrefillPlan prefill_plan(int B, int Hq, int Hkv, int Sq, int S, int d, bool qjl, bool extra, bool planes_only) {
-  PrefillPlan p{};
+  PrefillPlan base{};
   const int G = Hq / Hkv;
-  p.rows = prefill_rows_per_block(qjl);
-  p.qt = p.rows / G;
-  p.qtiles = (Sq - 1) / p.qt + 1;
-  p.splits = 1;
+  base.rows = prefill_rows_per_block(qjl);
+  base.qt = base.rows / G;
+  base.qtiles = (Sq - 1) / base.qt + 1;
+  base.splits = 1;
   const int64_t all = (int64_t)B * Hkv;
-  p.streams = (int)(all < 0x7fffffff ? all : 0x7fffffff);
-  if (!extra || S < 1) return p;
+  base.streams = (int)(all < 0x7fffffff ? all : 0x7fffffff);
+  if (!extra || S < 1) return base;
   const int tiles = (S - 1) / kPT + 1;   // (a size query may ask for any int)
+  // the plan that takes `streams` streams at a time, split where that leaves
+  // compute units idle (a split of four tiles at least)
+  auto of_streams = [&](int64_t streams) {
+    PrefillPlan p = base;
+    p.streams = (int)streams;
+    const int64_t blocks = p.qtiles * streams, most = tiles / 4;
+    const int64_t splits = kTargetBlocks / blocks < most ? kTargetBlocks / blocks : most;
+    if (splits > 1) {
+      p.splits = (int)splits;
+      p.part_rows = blocks * p.rows * splits;
+    }
+    return p;
+  };
+  // rounds of workgroups, one per compute unit, of n streams
+  auto rounds = [&](int64_t n, int splits) {
+    return splits > 1 ? 1.0 / splits : (double)((base.qtiles * n + kTargetBlocks - 1) / kTargetBlocks);
+  };
+  const PrefillPlan whole = of_streams(base.streams);
   // Decoding each tile once per call instead of once per row block pays from
   // some row blocks on (records are written and read back, 1 KB per token at
-  // d = 128). Whole calls, decoded once / per row block: d = 128 12 row blocks
-  // 103 / 117 us, 24 181 / 194 us, 64 against 131 072 tokens 16.9 / 18.7 ms, but
-  // 8 2.66 / 2.34 ms (256 streams) and 2.03 / 1.83 ms (256), 117 / 126 us (8
-  // streams); d = 64 6 387 / 454 us, 8 3.47 / 3.55 ms, 28 76 / 86 us, but 1
-  // 326 / 244 us.
-  p.stream_bytes = (int64_t)tiles * prefill_record_bytes(d);
-  p.planes = !qjl && (planes_only || p.qtiles >= (d == 128 ? 12 : 6)) && p.stream_bytes <= kPlaneBudget;
-  if (p.planes) {
-    // equal passes over the streams
-    const int64_t fit = kPlaneBudget / p.stream_bytes, passes = (all + fit - 1) / fit;
-    p.streams = (int)((all + passes - 1) / passes);
+  // d = 128). Whole calls, decoded once / per row block, us: d = 128, 8 streams
+  // against 4000 cached tokens (32 query / 8 kv heads) 12 row blocks 195 / 221, 8
+  // 128 / 132, 4 83 / 82, against none 72 / 73, 57 / 58, 43 / 42, 16 streams of 4
+  // against 16 000 393 / 357; d = 64 (14 / 2 heads), 16 streams against 4000 6 row
+  // blocks 128 / 143, 4 83 / 88, 2 58 / 58, 4 streams 57 / 54, 49 / 47, 43 / 39.
+  const int64_t stream_bytes = (int64_t)tiles * prefill_record_bytes(d), fit = kPlaneBudget / stream_bytes;
+  if (qjl || fit == 0 || !(planes_only || base.qtiles >= (d == 128 ? 12 : 6))) return whole;
+  // Where the records of all streams exceed the budget, the streams are taken
+  // in passes. A pass that ends on a part of a round of workgroups idles the
+  // rest, so the size of a pass is the one with the fewest rounds in all.
+  PrefillPlan best{};
+  double cost = 0.0;
+  for (int64_t n = fit < all ? fit : all; n >= 1; --n) {
+    PrefillPlan p = of_streams(n);
+    const double c = (double)(all / n) * rounds(n, p.splits) + (all % n ? rounds(all % n, p.splits) : 0.0);
+    if (!best.planes || c < cost) {
+      best = p;
+      best.planes = true;
+      best.stream_bytes = stream_bytes;
+      cost = c;
+    }
+    if (n == all || 2 * n <= fit) break;
   }
-  const int64_t blocks = (int64_t)p.qtiles * p.streams;
-  int64_t splits = kTargetBlocks / blocks;
-  if (splits > tiles / 4) splits = tiles / 4;   // a split of four tiles at least
-  if (splits > 1) {
-    p.splits = (int)splits;
-    p.part_rows = blocks * p.rows * splits;
-  }
-  return p;
+  // A round of workgroups that decode for themselves takes 1.06 (d = 64: 1.16) of
+  // one over records, and writing a stream's records takes 1 / 270 round (15 ns a
+  // tile against 4.1 us), so whole rounds of few row blocks decode for themselves
+  // too. Over records / per row block, 8 query / 8 kv heads, d = 128, 12 row
+  // blocks against 16 000 tokens: 32 streams 2.43 / 2.60 ms (2 rounds for 1.5),
+  // 64 streams 4.50 / 4.20; in passes, against 32 000 tokens (32 / 8 heads): 12 of
+  // 128 streams 21.1 / 16.9 ms (9 rounds for 6), of 512 70.0 / 64.6 (25 for 24), 24
+  // of 128 31.6 / 33.7 (12 for 12).
+  const double each = d == 128 ? 1.06 : 1.16;
+  const bool pays = (best.streams == all && whole.splits > 1) || cost + all / 270.0 <= each * rounds(all, whole.splits);
+  return planes_only || pays ? best : whole;
 }
 
 hipError_t launch_prefill_merge(const PrefillArgs &a, int stream0, int ns, int rows, hipStream_t s) {

@@ -80,6 +80,44 @@ def test_split_equals_whole(B, Hq, Hkv, Sq, q_start, d, causal, kind):
     _check(split, whole, vc if kind != "paged" else vc.to_contiguous(), R)
 
 
+# (B, Hq, Hkv, Sq, q_start, d, kind, streams of a pass): the records of all
+# streams exceed their 2 GiB
+PASSES = [(2, 32, 8, 1531, 138469, 128, "4", 10),
+          (2, 32, 8, 1531, 138469, 128, "paged", 10),
+          (2, 32, 8, 1531, 138469, 128, "mixed", 10),  # 14 streams of one pair of widths, 2 of the other
+          (4, 32, 8, 955, 138000, 64, "2", 17),
+          (1, 3, 3, 3071, 1500000, 64, "4", 1)]        # each split over 21 workgroups
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,q_start,d,kind,streams", PASSES)
+def test_passes_over_streams(B, Hq, Hkv, Sq, q_start, d, kind, streams):
+    """The records are written, read and joined again for each pass of streams."""
+    print(f"prefill passes {B} {Hq} {Hkv} Sq={Sq} q_start={q_start} d={d} {kind}", flush=True)
+    S = q_start + Sq
+    L = _lib.lib()
+    extra = (L.pqkv_prefill_workspace_preferred_bytes(B, Hq, Hkv, Sq, S, d, 0)
+             - L.pqkv_prefill_workspace_bytes(B, Hq, Hkv, Sq, S, d))
+    assert extra // (-(-S // 64) * (512 * d + 512)) == streams
+    R = torch.from_numpy(O.rotation_matrix(d, 42).astype(np.float32)).to(DEV)
+    caches = []
+    for i in range(2):
+        if kind == "paged":
+            c = quantizer.allocate_paged_cache(B, Hkv, d, 4, DEV, page_tokens=1024)
+        else:
+            bits = (4,) * (Hkv - 1) + (2,) if kind == "mixed" else int(kind)
+            c = quantizer.allocate_cache(B, Hkv, S, d, bits, DEV)
+        x = torch.randn(B, Hkv, S, d, generator=torch.Generator(DEV).manual_seed(i), device=DEV, dtype=torch.float16)
+        caches.append(quantizer.compress_pq(x, R, cache=c, start=0))
+        del x
+    kc, vc = caches
+    # queries that look at few keys, so that a stream's values show
+    q = (4 * torch.randn(B, Hq, Sq, d, generator=torch.Generator().manual_seed(S))).half().to(DEV)
+    got, want = _run(q, kc, vc, R, None, q_start, 1, True), _run(q, kc, vc, R, None, q_start, 1, False)
+    # logits reach 50: 2 (50 + 1) 2^-21 of a weight, and 2 2^-21 of max |v|, a norm of 20
+    assert float((got - want).abs().max()) <= 104 * 2.0 ** -21 * 20 and torch.isfinite(got).all()
+    assert float(want.abs().mean()) > 0.01
+
+
 def _call(q, kc, vc, R, jl, q_start, causal, ws):
     """pqkv_prefill_attn on a workspace of the caller's (a uint8 tensor), fp32 out."""
     B, Hq, Sq, d = q.shape
@@ -126,3 +164,31 @@ def test_decode_workspace_off_a_16_byte_boundary():
     ws = torch.empty(_lib.lib().pqkv_decode_workspace_bytes(B, Hq, Hkv, S, d) + 4, dtype=torch.uint8, device=DEV)
     got = [attention.decode_attention(q, kc, vc, R, jl_rot=jl, out_dtype=torch.float32, workspace=w) for w in (ws[:-4], ws[4:])]
     assert torch.equal(*got)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,q_start,d", [(1, 8, 2, 65, 1000, 128), (1, 8, 2, 801, 100, 128),
+                                                   (2, 14, 2, 300, 1003, 64)])
+@pytest.mark.parametrize("where", ["query", "key", "value"])
+@pytest.mark.parametrize("what", [float("inf"), float("nan"), 65504.0, 0.0])
+def test_values_at_the_ends_of_the_range(B, Hq, Hkv, Sq, q_start, d, where, what):
+    """Infinite, NaN, largest and zero queries and radii: NaN exactly where the
+    kernel that decodes per row block has it, the other rows as close as ever."""
+    print(f"prefill {where} {what} {B} {Hq} {Hkv} Sq={Sq} d={d}", flush=True)
+    S = q_start + Sq
+    R = torch.from_numpy(O.rotation_matrix(d, 42).astype(np.float32)).to(DEV)
+    kc, vc = (quantizer.compress_pq(_states(B, Hkv, S, d, 5 + i), R) for i in range(2))
+    q = (0.5 * torch.randn(B, Hq, Sq, d, generator=torch.Generator().manual_seed(S))).to(DEV)
+    if where == "query":
+        q[0, 0, 3], q[0, 1, 5, 2], q[-1, -1, Sq - 1, d - 1] = what, what, -what
+    else:
+        r = (kc if where == "key" else vc).blocks.view(B, Hkv, S, d // 32, 18)
+        for b, h, t in ((0, 0, S // 2), (B - 1, Hkv - 1, S - 1)):
+            r[b, h, t, :, :2] = torch.tensor([what], dtype=torch.float16).view(torch.uint8).to(DEV)
+    got, want = _run(q, kc, vc, R, None, q_start, 1, True), _run(q, kc, vc, R, None, q_start, 1, False)
+    nan = torch.isnan(want)
+    assert torch.equal(torch.isnan(got), nan) and not torch.isinf(got).any()
+    assert nan.any() or np.isfinite(what)
+    # (a largest query or key radius makes logits whose 2^-21 moves a weight freely)
+    if not nan.all() and not (what == 65504.0 and where != "value"):
+        size = 65504.0 if what == 65504.0 else float(quantizer.dequantize(vc, None, torch.float32).nan_to_num(0, 0, 0).abs().max())
+        assert float((got - want)[~nan].abs().max()) <= 20 * 2.0 ** -21 * size * np.sqrt(d)
