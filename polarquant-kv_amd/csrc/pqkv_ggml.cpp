@@ -258,12 +258,15 @@ namespace {
 
 // From these query rows per sequence and this work (query rows x kv heads x
 // tokens x d) on, the cache is decoded once per call instead of streamed once
-// per row. Whole calls, streamed / decoded once, us: 32 query / 8 kv heads, d =
-// 128, 64 rows against 4096 tokens (2^28) 75 / 69, 512 against 512 (2^28) 150 /
+// per row; from twice that work where one row block is all there is, whose
+// tokens are split over so many workgroups that joining them takes as long as
+// the rest. Whole calls, streamed / decoded once, us: 32 query / 8 kv heads, d =
+// 128, 64 rows against 4096 tokens (2^28) 76 / 64, 512 against 512 (2^28) 150 /
 // 71, but 2 x 16 against 4096 (2^27) 46 / 74; 32 / 32 heads 64 against 4096 207
-// / 104, but 2 x 16 (2^29) 115 / 187, 64 against 512 (2^27) 48 / 56; 64 / 8
-// heads 64 against 4096 102 / 75; d = 64, 14 / 2 heads, 512 against 4096 (2^28)
-// 116 / 68, against 512 39 / 42.
+// / 104, but 2 x 16 (2^29) 115 / 187, 64 against 512 (2^27) 48 / 56; 4 / 4 heads
+// 64 against 8192 (2^28) 64 / 58, 65 against 8192 85 / 59; 1 / 1 head 64 against
+// 32 768 (2^28) 58 / 70; d = 64, 14 / 2 heads, 512 against 4096 (2^28) 116 / 68,
+// against 512 39 / 42; 2 / 2 heads 64 against 32 768 (2^28) 72 / 58.
 constexpr int kManyRows = 64;
 constexpr int64_t kManyWork = (int64_t)1 << 28;
 
@@ -316,10 +319,10 @@ int fa_shape(const polarquant_state *st, const int64_t ne_q[4], const int64_t ne
   f->many = false;
   f->many_bytes = f->bytes;
   if (f->n_seq > 0 && f->n_q >= kManyRows && f->Hq > 0 && f->n_kv > 0 && f->n_kv % 4 == 0 &&
-      (double)rows * f->Hkv * f->n_kv * d >= (double)kManyWork &&
       f->Hq / f->Hkv <= pqkv::prefill_rows_per_block(false)) {
     f->plan = pqkv::prefill_plan(f->n_seq, f->Hq, f->Hkv, f->n_q, f->n_kv, d, false, true, true);
-    f->many = f->plan.planes;
+    const bool one_block = (int64_t)f->n_seq * f->Hkv * f->plan.qtiles == 1;
+    f->many = f->plan.planes && (double)rows * f->Hkv * f->n_kv * d >= (double)kManyWork * (one_block ? 2 : 1);
     const size_t arr = ((size_t)rows * f->Hq * d * 4 + 255) & ~(size_t)255;
     f->o_off = arr;                              // queries, output, partials and records
     f->extra_off = 2 * arr;
