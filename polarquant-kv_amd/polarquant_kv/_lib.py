@@ -179,6 +179,18 @@ def require_device(*tensors) -> None:
             raise ValueError("GPU entry points take device tensors (the hot path has no CPU fallback)")
 
 
+def workspace(best: int, least: int, device):
+    """A workspace of `best` bytes, the size a call is fastest with, or of
+    `least`, the smallest it takes, where the device has no room for that."""
+    import torch
+    try:
+        return torch.empty(max(best, 1), dtype=torch.uint8, device=device)
+    except torch.cuda.OutOfMemoryError:
+        if best <= least:
+            raise
+    return torch.empty(max(least, 1), dtype=torch.uint8, device=device)
+
+
 def ptr_array(tensors):
     """Host array of the tensors' device pointers (for the segment arrays)."""
     return (c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])

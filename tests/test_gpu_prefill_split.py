@@ -192,3 +192,27 @@ def test_values_at_the_ends_of_the_range(B, Hq, Hkv, Sq, q_start, d, where, what
     if not nan.all() and not (what == 65504.0 and where != "value"):
         size = 65504.0 if what == 65504.0 else float(quantizer.dequantize(vc, None, torch.float32).nan_to_num(0, 0, 0).abs().max())
         assert float((got - want)[~nan].abs().max()) <= 20 * 2.0 ** -21 * size * np.sqrt(d)
+
+
+@pytest.mark.parametrize("paged", [False, True])
+def test_no_room_for_the_preferred_workspace(paged, monkeypatch):
+    """A device too full for the preferred workspace runs the base plan."""
+    B, Hq, Hkv, Sq, q_start, d = 1, 8, 2, 801, 100, 128
+    S = q_start + Sq
+    R = torch.from_numpy(O.rotation_matrix(d, 42).astype(np.float32)).to(DEV)
+    caches = [quantizer.allocate_paged_cache(B, Hkv, d, 4, DEV, page_tokens=64) if paged else
+              quantizer.allocate_cache(B, Hkv, S, d, 4, DEV) for _ in range(2)]
+    kc, vc = (quantizer.compress_pq(_states(B, Hkv, S, d, 5 + i), R, cache=c, start=0) for i, c in enumerate(caches))
+    q = (0.5 * torch.randn(B, Hq, Sq, d, generator=torch.Generator().manual_seed(S))).half().to(DEV)
+    want = _run(q, kc, vc, R, None, q_start, 1, False)
+    base, real, refused = _lib.lib().pqkv_prefill_workspace_bytes(B, Hq, Hkv, Sq, S, d), torch.empty, []
+
+    def empty(*size, **kw):
+        if len(size) == 1 and size[0] > base:
+            refused.append(size[0])
+            raise torch.cuda.OutOfMemoryError("out of memory")
+        return real(*size, **kw)
+
+    monkeypatch.setattr(torch, "empty", empty)
+    got = attention.prefill_attention(q, kc, vc, R, q_start, out_dtype=torch.float32)
+    assert refused and torch.equal(got, want)

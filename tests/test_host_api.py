@@ -233,3 +233,22 @@ def test_paged_cache_tables_on_the_host():
     assert a.capacity == 256
     with pytest.raises(ValueError):
         a.ensure(257)
+
+
+def test_workspace_falls_back_to_the_smallest(monkeypatch):
+    """No room for the faster plan's workspace: the call gets the smallest one;
+    no room for that either: the error."""
+    real, room = torch.empty, 1000
+
+    def empty(n, **kw):
+        if n > room:
+            raise torch.cuda.OutOfMemoryError("out of memory")
+        return real(n, **kw)
+
+    monkeypatch.setattr(torch, "empty", empty)
+    assert _lib.workspace(900, 100, "cpu").numel() == 900
+    assert _lib.workspace(5000, 1000, "cpu").numel() == 1000
+    assert _lib.workspace(0, 0, "cpu").numel() == 1
+    for best, least in ((5000, 1001), (1001, 1001)):
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            _lib.workspace(best, least, "cpu")
