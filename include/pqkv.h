@@ -541,11 +541,18 @@ int pqkv_ggml_cpy_pq4(const polarquant_state *st, const void *src, int src_type,
  *   head h reads kv head h / (Hq / Hkv); a row whose tokens are all masked
  *   (-inf) is 0. max_bias and logit_softcap must be 0 (PQKV_ERR_UNSUPPORTED
  *   otherwise: a backend's supports_op declines those). d = st->head_dim.
- * The workspace (pqkv_ggml_flash_attn_ext_pq4_workspace_bytes, 0 for an
- * invalid shape) needs no initialisation. Several query rows per sequence
- * (n_q > 1) each stream the whole key / value sequence. */
+ * The workspace (at least pqkv_ggml_flash_attn_ext_pq4_workspace_bytes, 0
+ * for an invalid shape) needs no initialisation. With that size every query
+ * row streams the whole key / value sequence; with
+ * pqkv_ggml_flash_attn_ext_pq4_workspace_preferred_bytes prompts of many rows
+ * run over the cache's tiles decoded once per call (about 1 KB per cached
+ * token and kv head at d = 128, at most 2 GiB, and the rotated queries and
+ * outputs; the same size where that does not pay). A mask is read four values
+ * at a time there: 8-byte aligned rows, else the rows are streamed. */
 size_t pqkv_ggml_flash_attn_ext_pq4_workspace_bytes(const polarquant_state *st, const int64_t ne_q[4],
                                                     const int64_t ne_k[4]);
+size_t pqkv_ggml_flash_attn_ext_pq4_workspace_preferred_bytes(const polarquant_state *st, const int64_t ne_q[4],
+                                                              const int64_t ne_k[4]);
 int pqkv_ggml_flash_attn_ext_pq4(const polarquant_state *st, const float *q, const int64_t ne_q[4],
                                  const size_t nb_q[4], const void *k, const int64_t ne_k[4], const size_t nb_k[4],
                                  const void *v, const int64_t ne_v[4], const size_t nb_v[4], const void *mask,

@@ -338,6 +338,12 @@ extern "C" {
 size_t pqkv_ggml_flash_attn_ext_pq4_workspace_bytes(const polarquant_state *st, const int64_t ne_q[4],
                                                     const int64_t ne_k[4]) {
   FaShape f;
+  return fa_shape(st, ne_q, ne_k, &f) == PQKV_OK ? f.bytes : 0;
+}
+
+size_t pqkv_ggml_flash_attn_ext_pq4_workspace_preferred_bytes(const polarquant_state *st, const int64_t ne_q[4],
+                                                              const int64_t ne_k[4]) {
+  FaShape f;
   return fa_shape(st, ne_q, ne_k, &f) == PQKV_OK ? f.many_bytes : 0;
 }
 

@@ -116,6 +116,7 @@ SIGNATURES = {
     "pqkv_ggml_dequantize_row_pq4": (None, [c_void_p, c_void_p, c_int64]),
     "pqkv_ggml_cpy_pq4": (c_int, [c_void_p, c_void_p, c_int, c_int64_p, c_size_p, c_void_p, c_size_p, c_void_p]),
     "pqkv_ggml_flash_attn_ext_pq4_workspace_bytes": (c_size_t, [c_void_p, c_int64_p, c_int64_p]),
+    "pqkv_ggml_flash_attn_ext_pq4_workspace_preferred_bytes": (c_size_t, [c_void_p, c_int64_p, c_int64_p]),
     "pqkv_ggml_flash_attn_ext_pq4": (c_int, [c_void_p, c_void_p, c_int64_p, c_size_p, c_void_p, c_int64_p, c_size_p,
                                              c_void_p, c_int64_p, c_size_p, c_void_p, c_int64_p, c_size_p,
                                              c_float, c_float, c_float, c_void_p, c_void_p, c_size_t,

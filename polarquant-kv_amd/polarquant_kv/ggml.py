@@ -164,11 +164,11 @@ def flash_attn_ext(state: State, q, k, v, mask=None, scale: float = 1.0, max_bia
     ns, Hq, n_q = q.shape[0], q.shape[1], q.shape[2]
     out = torch.empty((ns, n_q, Hq, d), dtype=torch.float32, device=q.device)
     L = _lib.lib()
-    ws_bytes = L.pqkv_ggml_flash_attn_ext_pq4_workspace_bytes(state.ptr, qne, kne)
-    ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=q.device)
+    ws = _lib.workspace(L.pqkv_ggml_flash_attn_ext_pq4_workspace_preferred_bytes(state.ptr, qne, kne),
+                        L.pqkv_ggml_flash_attn_ext_pq4_workspace_bytes(state.ptr, qne, kne), q.device)
     _lib.check(L.pqkv_ggml_flash_attn_ext_pq4(state.ptr, q.data_ptr(), qne, qnb, k.data_ptr(), kne, knb,
                                               v.data_ptr(), vne, vnb, mp, mne, mnb, float(scale), float(max_bias),
-                                              float(logit_softcap), out.data_ptr(), ws.data_ptr(), ws_bytes,
+                                              float(logit_softcap), out.data_ptr(), ws.data_ptr(), ws.numel(),
                                               _lib.stream_of(q)))
     return out
 

@@ -202,3 +202,18 @@ def test_flash_attn_ext_rejects_bad_arguments_before_any_launch():
     mnb = _arr4(_lib.c_size_4, [2, 2 * n_kv, 2 * n_kv, 2 * n_kv])
     assert call(mask=0x6000, mne=mne, mnb=mnb) == _lib.ERR_INVALID
     assert call(wsb=ws - 1) == _lib.ERR_WORKSPACE
+
+
+@pytest.mark.parametrize("d,n_q,Hq,Hkv,n_kv,more", [(128, 512, 32, 8, 4096, True), (128, 1, 32, 8, 4096, False),
+                                                    (128, 63, 32, 8, 4096, False), (128, 64, 1, 1, 32768, False),
+                                                    (128, 512, 32, 8, 4095, False), (64, 512, 14, 2, 4096, True)])
+def test_flash_attn_ext_workspace_sizes(d, n_q, Hq, Hkv, n_kv, more):
+    """The least workspace does not grow with the tiles decoded once per call;
+    the preferred one asks for them where the call would use them."""
+    L, st = _lib.lib(), _fake_state(d=d)
+    qne, kne = _arr4(_lib.c_int64_4, [d, n_q, Hq, 1]), _arr4(_lib.c_int64_4, [d, n_kv, Hkv, 1])
+    least = L.pqkv_ggml_flash_attn_ext_pq4_workspace_bytes(ctypes.byref(st), qne, kne)
+    best = L.pqkv_ggml_flash_attn_ext_pq4_workspace_preferred_bytes(ctypes.byref(st), qne, kne)
+    tiles = (n_kv + 63) // 64 * (512 * d + 512) * Hkv
+    assert least > 0
+    assert best >= least + tiles // 2 if more else best == least
