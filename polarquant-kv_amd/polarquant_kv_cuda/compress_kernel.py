@@ -102,8 +102,11 @@ def _compress_rows(x: torch.Tensor, R: torch.Tensor, n_bits: int, group_size: in
     code = {torch.float16: _lib.F16, torch.float32: _lib.F32, torch.bfloat16: _lib.BF16}[x.dtype]
     Rf = R.to(device=x.device, dtype=torch.float32).contiguous()
     resid = torch.empty(n, d, dtype=torch.float32, device=x.device) if jl_matrix is not None else None
-    # the matrix-core encoder reads R alone; the general one is faster with R^T
-    Rt = None if d in (64, 128) and group_size in (8, 16, 32, 64, 128) and x.data_ptr() % 16 == 0 else _transposed(Rf)
+    # the matrix-core encoder reads R alone; the general one, which takes every
+    # other form, is faster with R^T
+    mfma = (d in (64, 128) and group_size in (8, 16, 32, 64, 128) and group_size <= d
+            and all(t.data_ptr() % 16 == 0 for t in (x, Rf, out["codes"])))
+    Rt = None if mfma else _transposed(Rf)
     _lib.check(lib.pqkv_group_gpu_compress(x.data_ptr(), code, Rf.data_ptr(), _lib.ptr(Rt), n, d,
                                            n_bits, group_size, out["radius"].data_ptr(), out["codes"].data_ptr(),
                                            out["mins"].data_ptr(), out["scales"].data_ptr(), _lib.F16,

@@ -9,6 +9,7 @@ import torch
 
 from oracle import oracle as O
 from polarquant_kv import _lib
+from polarquant_kv_cuda.compress_kernel import compress_gpu
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -97,3 +98,29 @@ def test_special_values(d, identity):
     R = torch.eye(d) if identity else torch.from_numpy(O.rotation_matrix(d, 42).astype(np.float32))
     for gs in (8, 16, d):
         _both(x.to(DEV), R.to(DEV), 4, gs, _lib.F32, True)
+
+
+@pytest.mark.parametrize("d,gs,off,transposed", [(128, 32, 0, False), (64, 64, 0, False), (128, 32, 1, True),
+                                                 (128, 12, 0, True), (96, 32, 0, True)])
+def test_general_kernel_gets_the_transposed_rotation(d, gs, off, transposed, monkeypatch):
+    """compress_gpu transposes R exactly where the general kernel runs: without
+    R^T its lanes read a row of R each."""
+    R = torch.from_numpy(np.linalg.qr(np.random.default_rng(3).standard_normal((d, d)))[0].astype(np.float32)).to(DEV)
+    flat = torch.empty(d * d + 8, device=DEV)
+    Ro = flat[off:off + d * d].view(d, d)
+    Ro.copy_(R)
+    x = torch.randn(1, 2, 33, d, generator=torch.Generator().manual_seed(d)).to(DEV)
+    lib, seen = _lib.lib(), []
+
+    class Spy:
+        def __getattr__(self, name):
+            f = getattr(lib, name)
+            if name != "pqkv_group_gpu_compress":
+                return f
+            return lambda *a: seen.append(a[3] is not None) or f(*a)
+
+    monkeypatch.setattr(_lib, "_lib", Spy())
+    got, want = compress_gpu(x, Ro, 4, gs), compress_gpu(x, R, 4, gs)
+    assert seen[0] == transposed
+    for f in ("radius", "quantized_direction", "group_mins", "group_scales"):
+        assert torch.equal(getattr(got, f), getattr(want, f)), f
