@@ -506,7 +506,7 @@ __global__ void __launch_bounds__(256) encode_exact_kernel(EncodeArgs a) {
         if (base + t < n) {
           const uint32_t cw = cs[t][j & 63];
           const int code = D == 128 ? ((j < 64) ? (cw & 15) : (cw >> 4)) : (cw & 15);
-          xs[t][j] = ys[t][j] - rs[t] * cb[code];
+          xs[t][j] = __builtin_fmaf(-rs[t], cb[code], ys[t][j]);   // (as encode_chain_kernel)
         }
       }
       __syncthreads();

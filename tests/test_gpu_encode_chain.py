@@ -57,12 +57,8 @@ def test_blocks_and_signs(d, bits, dtype, rows, n, pad):
     for p in (None, P):
         got, want = _encode(x, rows, d, bits, R, p, cb, pad), _encode(off, rows, d, bits, R, p, cb, pad)
         assert torch.equal(got[0], want[0])
-        if p is not None:
-            # each side sums P_rot e as the same chain; the residual is the
-            # same fused multiply-add up to the general kernel's two roundings
-            diff = (got[1] ^ want[1]).flatten()
-            bits_off = sum(int(((diff >> k) & 1).sum()) for k in range(8))
-            assert bits_off <= 1e-5 * diff.numel() * 8 + 2
+        if p is not None:   # the same chains of one fused multiply-add per residual
+            assert torch.equal(got[1], want[1])
 
 
 @pytest.mark.parametrize("d", [64, 128])
