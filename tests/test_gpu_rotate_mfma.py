@@ -152,3 +152,33 @@ def test_dequantize_of_empty_and_expanded_caches(bits):
         heads = quantizer.allocate_cache(2, 3, cap, d, bits, DEV)
         heads.blocks, heads.seq_len = one.blocks[:, :1].expand(2, 3, -1, -1), S
         assert torch.equal(quantizer.dequantize(heads, R, torch.float32), want[:, :1].expand(2, 3, -1, -1))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("inverse", [0, 1])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_rotate_bits_past_one_resident_round(d, inverse, dtype):
+    """About 2.5 steps per workgroup (four of them per compute unit, 32 vectors a
+    step, 64 at d = 64) and a remainder, against small launches."""
+    n = (82000 if d == 128 else 164000) + 7
+    print(f"rotate steady state d={d} inverse={inverse} {dtype}", flush=True)
+    assert n > 2 * 4 * torch.cuda.get_device_properties(0).multi_processor_count * (32 if d == 128 else 64)
+    R = torch.from_numpy(O.rotation_matrix(d, 42).astype(np.float32)).to(DEV)
+    x = torch.randn(n, d, generator=torch.Generator(DEV).manual_seed(d), device=DEV).to(dtype)
+    many = _rotate(x, R, inverse, torch.empty(n, d, device=DEV))
+    few = torch.empty(n, d, device=DEV)
+    for i in range(0, n, 2000):
+        _rotate(x[i:i + 2000], R, inverse, few[i:i + 2000])
+    assert torch.equal(_bits(many), _bits(few))
+
+
+@pytest.mark.parametrize("d,bits", [(64, 2), (64, 4), (128, 2), (128, 4)])
+def test_dequantize_bits_past_one_resident_round(d, bits):
+    """The same for rows of a cache longer than its valid positions."""
+    B, H, S, cap = 3, 4, 6841 if d == 128 else 13677, 13700
+    print(f"dequantize steady state d={d} bits={bits}", flush=True)
+    cache, rows = _block_cache(B, H, S, cap, d, bits)
+    R = torch.from_numpy(O.rotation_matrix(d, 42).astype(np.float32)).to(DEV)
+    for dtype in (torch.float16, torch.float32):
+        got = quantizer.dequantize(cache, R, dtype).reshape(-1, d)
+        assert torch.equal(_bits(got), _bits(_in_chunks(rows, R, cache.codebooks, bits, d, dtype, 1000)))
