@@ -281,10 +281,12 @@ REPEAT = 20
 
 def kernel_means(torch, _lib, fn, steps, names, repeat=REPEAT):
     """Live per-launch kernel times: with the library's profiling on, every
-    bracketed kernel of a step (rotation, split, merge, encoder, prefill) is
-    launched `repeat` times back to back between two hipEvents on its launch
-    stream (the kernels are idempotent), for `steps` steps. Returns, per
-    name, the mean ms per launch times the launches one plain step makes."""
+    bracketed kernel of a step (a decode's rotation, split, merge, encoder,
+    prefill) is launched `repeat` times back to back between two hipEvents on
+    its launch stream (the kernels are idempotent), for `steps` steps; the
+    rotations around a prefill and of the ggml queries are launched once.
+    Returns, per name, the mean ms per launch times the launches one plain step
+    makes."""
     _lib.profile_repeat(repeat)
     _lib.profile_enable(True)
     _lib.profile_collect("")
@@ -296,7 +298,9 @@ def kernel_means(torch, _lib, fn, steps, names, repeat=REPEAT):
     res = {}
     for n in names:
         ms, launches = _lib.profile_collect(n)
-        per_step = launches / (repeat * steps)           # launches of this family in one plain step
+        per_step = launches / steps                      # launches of this family in one plain step ...
+        if per_step >= repeat:
+            per_step /= repeat                           # ... made `repeat` times each
         res[n] = ms / max(launches, 1) * per_step
     _lib.profile_enable(False)
     _lib.profile_repeat(1)
@@ -875,7 +879,8 @@ def run_config5(args) -> int:
                    "global_batch": B, "seq_len": S, "parallelism": "single GPU"},
         "roofline": {"bound": "mfma", "achieved": round(kern_tflops, 2), "peak": MFMA_F16_PEAK_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(kern_tflops / MFMA_F16_PEAK_TFLOPS, 4), "traffic": None,
-                     "kernel": "prefill_mfma_kernel<128,4,4,false>", "kernel_ms": round(km["prefill_attn"], 4),
+                     "kernel": "plane_decode_kernel<128,4,4> and prefill_planes_kernel<128,false>",
+                     "kernel_ms": round(km["prefill_attn"], 4),
                      "kernel_ms_source": KSRC,
                      "flops_per_launch": flops,
                      "note": "fp32-grade products cost 3 fp16 MFMAs each: this arithmetic tops out at 1/3"},
