@@ -8,7 +8,7 @@
 // against fmaf over 128-long chains (12.8 M outputs: normal data, exponents
 // spread over 2^+-40, products and operands in the subnormal range, fp16
 // values): every bit equal. So a chain of these instructions over ascending k
-// gives the chain's bits, at 142-147 TFLOP/s measured (all CUs) without vector
+// gives the chain's bits, at 142-154 TFLOP/s measured (all CUs) without vector
 // ALU work, where the vector ALU reaches 109-111 TFLOP/s of FMAs alone and
 // 62 TFLOP/s in a register-blocked kernel that has to feed them from LDS
 // (v_mfma_f32_16x16x4_f32 rounds alike but reaches 126-129 TFLOP/s).

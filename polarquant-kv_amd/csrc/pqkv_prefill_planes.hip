@@ -34,13 +34,16 @@
 // split) takes its share of the row block's tiles and writes an unnormalised
 // partial; prefill_merge_kernel joins them.
 //
-// Bound by the matrix cores at the card's power limit. 64 query / 8 kv heads,
-// 2048 tokens against 131 072 (26.6 TFLOP of products): 16.9 ms in all against
-// 18.85 for decoding per row block, 1575 TFLOP/s, the matrix cores busy 67 %
-// of the cycles at 1.82 GHz; a library product of two 8192 x 8192 fp16 matrices
-// reaches 1330 TFLOP/s on the same card. v_mfma_f32_32x32x16_f16 products (half
-// the operand reads) draw more: 18.6 ms. The decode kernel takes 0.25 ms of it
-// (1.07 GB of records, 4.3 TB/s).
+// Bound by the matrix stage: 64 query / 8 kv heads, 2048 tokens against 131 072
+// (26.6 TFLOP of products) take 16.9-18.5 ms box to box, 18.85-20.4 for decoding
+// per row block; at 18.5 ms 1440 TFLOP/s, the matrix cores busy 71 % of the
+// cycles and a quarter of the wave cycles waiting (the barriers between the
+// groups' stages), at 1.89 GHz where short kernels run at 2.1-2.4, memory at 0.12
+// TB/s and no bank conflicts. v_mfma_f32_16x16x32_f16 alone reaches 2390 TFLOP/s
+// in a burst of 0.4 ms, a library product of two 8192 x 8192 fp16 matrices 1323.
+// v_mfma_f32_32x32x16_f16 products (half the operand reads) take 18.6 ms where
+// these take 16.9. The decode kernel takes 0.25 ms of it (1.10 GB of records, 4.4
+// TB/s).
 #include <type_traits>
 
 #include "pqkv_device.h"
@@ -172,9 +175,10 @@ __global__ void __launch_bounds__(256) plane_decode_kernel(const PrefillArgs a, 
 // largest value radius so far), since they are fp32 there and the results too. 512
 // query rows (32 query / 8 kv heads, d = 128) against 4096 tokens: 143 us a
 // call, 461 for the split decode kernel, which streams the cache once per row;
-// the error against 64 bits is 6.4e-7 (8.1e-7 there). Bound by the matrix cores
-// and the mask's loads; the 40 bytes a lane spills at d = 128 buy the tile sums
-// (1-2 %).
+// the error against 64 bits is 6.4e-7 (8.1e-7 there). 123 us of it are this
+// kernel, 845 TFLOP/s executed, its waves waiting for 44 % of their cycles (16
+// tiles a workgroup: set-up, mask loads, barriers); the 40 bytes a lane spills at
+// d = 128 buy the tile sums (1-2 %).
 template <int D, bool GG>
 __global__ void __launch_bounds__(kPW * 64, 1)
     prefill_planes_kernel(const PrefillArgs a, const uint8_t *planes, int64_t stream_bytes, int stream0, int ns) {
