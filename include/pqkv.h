@@ -341,9 +341,11 @@ int pqkv_soa_attn_generic(const float *q_rot, const uint8_t *k_codes, const floa
  * pqkv_decode_attn. */
 size_t pqkv_prefill_workspace_bytes(int B, int Hq, int Hkv, int Sq, int S, int d);
 /* The workspace with which pqkv_prefill_attn (and _paged) is fastest: at least
- * pqkv_prefill_workspace_bytes; for long chunks (without QJL) also room for
- * the cache's tiles decoded once per call, about 1 KB per cached token and kv
- * head at d = 128, at most 2 GiB. Any size from the smaller one on is accepted. */
+ * pqkv_prefill_workspace_bytes; for few query rows also room for the partials of
+ * a split (at most 34 MB), for long chunks (without QJL) for the cache's tiles
+ * decoded once per call, about 1 KB per cached token and kv head at d = 128, at
+ * most 2 GiB. Any size from the smaller one on is accepted (the room beyond it
+ * is used where all of it is there, on a 16-byte boundary). */
 size_t pqkv_prefill_workspace_preferred_bytes(int B, int Hq, int Hkv, int Sq, int S, int d, int qjl);
 
 int pqkv_prefill_attn(const void *q, int q_dtype, const float *R,

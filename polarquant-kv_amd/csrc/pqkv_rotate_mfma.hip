@@ -73,19 +73,14 @@ struct StridedSource {
   const float *x;
   int64_t s_q, s_h, s_s;
   int n_q, Hq;
-  struct Raw { float4_t a, b; };
+  using Raw = typename F32Source<D>::Raw;
   __device__ __forceinline__ Raw load(int64_t v, int j8) const {
     const int64_t rest = v / Hq, h = v - rest * Hq;
     const int64_t sq = rest / n_q, iq = rest - sq * n_q;
-    const float4_t *p = (const float4_t *)(x + sq * s_s + h * s_h + iq * s_q + 8 * j8);
-    return {p[0], p[1]};
+    return F32Source<D>{x + sq * s_s + h * s_h + iq * s_q}.load(0, j8);
   }
-  __device__ __forceinline__ void values(const Raw &w, int, const float *, float (&o)[8]) const {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      o[e] = w.a[e];
-      o[4 + e] = w.b[e];
-    }
+  __device__ __forceinline__ void values(const Raw &w, int j8, const float *cb, float (&o)[8]) const {
+    F32Source<D>{x}.values(w, j8, cb, o);
   }
 };
 // Block-encoded vectors: r16 c[code]. A piece is one dword of qs (4-bit) or
