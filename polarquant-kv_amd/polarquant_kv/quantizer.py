@@ -222,27 +222,30 @@ def dequantize(cache: PQCache, rotation_matrix: torch.Tensor | None, out_dtype=t
     lib = _lib.lib()
     stream = _lib.stream_of(out)
     code = _lib.dtype_code(out_dtype)
+    blocks, dst, es, r = cache.blocks.data_ptr(), out.data_ptr(), out.element_size(), R.data_ptr()
 
-    def rows(blocks, stride, cb, bits, dst, dst_stride, n):
+    def rows(src, stride, cb, bits, to, to_stride, n):
         """n rows of S vectors `stride` bytes apart; a launch takes rows that
         do not overlap, those of an expanded cache go one by one."""
         one_launch = n == 1 or stride >= S * vector_bytes(d, bits)
         for i in range(1 if one_launch else n):
-            _lib.check(lib.pqkv_dequantize_rows(blocks + i * stride, stride, cb.data_ptr(), bits, R.data_ptr(),
-                                                dst[i].data_ptr(), code, dst_stride, n if one_launch else 1, S, d, stream))
+            _lib.check(lib.pqkv_dequantize_rows(src + i * stride, stride, cb, bits, r, to + i * to_stride * es, code,
+                                                to_stride, n if one_launch else 1, S, d, stream))
 
     if not cache.mixed:
         # every (batch, head) row of the cache, S_max vectors apart, in one
         # launch (one per batch row where the batch stride is its own)
         sb, sh = cache.blocks.stride(0), cache.blocks.stride(1)
         n, batches = (B * H, 1) if sb == H * sh else (H, B)
+        cb = cache.codebooks.data_ptr()
         for b in range(batches):
-            rows(cache.blocks[b].data_ptr(), sh, cache.codebooks, cache.n_bits, out[b:].flatten(0, 1), S * d, n)
+            rows(blocks + b * sb, sh, cb, cache.n_bits, dst + b * H * S * d * es, S * d, n)
         return out
     for h, bits in enumerate(cache.head_bits()):
         # one head of every batch row per launch
         cb = cache.codebooks[h] if cache.codebooks.dim() == 2 else cache.codebooks
-        rows(cache.blocks.data_ptr() + cache.head_offset(h), cache.blocks.stride(0), cb, bits, out[:, h], H * S * d, B)
+        rows(blocks + cache.head_offset(h), cache.blocks.stride(0), cb.data_ptr(), bits, dst + h * S * d * es,
+             H * S * d, B)
     return out
 
 
