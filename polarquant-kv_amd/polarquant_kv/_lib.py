@@ -180,16 +180,17 @@ def require_device(*tensors) -> None:
             raise ValueError("GPU entry points take device tensors (the hot path has no CPU fallback)")
 
 
-def workspace(best: int, least: int, device):
+def workspace(best: int, least, device):
     """A workspace of `best` bytes, the size a call is fastest with, or of
-    `least`, the smallest it takes, where the device has no room for that."""
+    least(), the smallest it takes, where the device has no room for that."""
     import torch
     try:
-        return torch.empty(max(best, 1), dtype=torch.uint8, device=device)
+        return torch.empty(best or 1, dtype=torch.uint8, device=device)
     except torch.cuda.OutOfMemoryError:
-        if best <= least:
+        n = least()
+        if best <= n:
             raise
-    return torch.empty(max(least, 1), dtype=torch.uint8, device=device)
+    return torch.empty(n or 1, dtype=torch.uint8, device=device)
 
 
 def ptr_array(tensors):

@@ -213,7 +213,7 @@ def prefill_attention(query: torch.Tensor, keys: PQCache, values: PQCache, rotat
     S = keys.seq_len
     shape = (B, Hq, Hkv, Sq, max(S, 1), d)
     ws = _lib.workspace(lib.pqkv_prefill_workspace_preferred_bytes(*shape, int(jl_rot is not None)),
-                        lib.pqkv_prefill_workspace_bytes(*shape), q.device)
+                        lambda: lib.pqkv_prefill_workspace_bytes(*shape), q.device)
     mixed = keys.mixed or values.mixed
     kbits = _lib.int_array(keys.head_bits()) if mixed else None
     vbits = _lib.int_array(values.head_bits()) if mixed else None
@@ -244,7 +244,7 @@ def _prefill_paged(query, keys, values, rotation_matrix, q_start, causal, scale,
     S = keys.seq_len
     shape = (B, Hq, Hkv, Sq, max(S, 1), d)
     ws = _lib.workspace(lib.pqkv_prefill_workspace_preferred_bytes(*shape, int(jl_rot is not None)),
-                        lib.pqkv_prefill_workspace_bytes(*shape), q.device)
+                        lambda: lib.pqkv_prefill_workspace_bytes(*shape), q.device)
     if jl_rot is not None and keys.sign_table is None:
         raise ValueError("QJL correction requested but the key cache has no signs")
     P = None if jl_rot is None else jl_rot.to(torch.float32).contiguous()

@@ -165,7 +165,7 @@ def flash_attn_ext(state: State, q, k, v, mask=None, scale: float = 1.0, max_bia
     out = torch.empty((ns, n_q, Hq, d), dtype=torch.float32, device=q.device)
     L = _lib.lib()
     ws = _lib.workspace(L.pqkv_ggml_flash_attn_ext_pq4_workspace_preferred_bytes(state.ptr, qne, kne),
-                        L.pqkv_ggml_flash_attn_ext_pq4_workspace_bytes(state.ptr, qne, kne), q.device)
+                        lambda: L.pqkv_ggml_flash_attn_ext_pq4_workspace_bytes(state.ptr, qne, kne), q.device)
     _lib.check(L.pqkv_ggml_flash_attn_ext_pq4(state.ptr, q.data_ptr(), qne, qnb, k.data_ptr(), kne, knb,
                                               v.data_ptr(), vne, vnb, mp, mne, mnb, float(scale), float(max_bias),
                                               float(logit_softcap), out.data_ptr(), ws.data_ptr(), ws.numel(),

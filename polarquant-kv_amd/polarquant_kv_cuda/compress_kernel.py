@@ -105,7 +105,7 @@ def _compress_rows(x: torch.Tensor, R: torch.Tensor, n_bits: int, group_size: in
     # the matrix-core encoder reads R alone; the general one, which takes every
     # other form, is faster with R^T
     mfma = (d in (64, 128) and group_size in (8, 16, 32, 64, 128) and group_size <= d
-            and all(t.data_ptr() % 16 == 0 for t in (x, Rf, out["codes"])))
+            and (x.data_ptr() | Rf.data_ptr() | out["codes"].data_ptr()) % 16 == 0)
     Rt = None if mfma else _transposed(Rf)
     _lib.check(lib.pqkv_group_gpu_compress(x.data_ptr(), code, Rf.data_ptr(), _lib.ptr(Rt), n, d,
                                            n_bits, group_size, out["radius"].data_ptr(), out["codes"].data_ptr(),
